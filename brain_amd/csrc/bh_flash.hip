@@ -1,0 +1,458 @@
+// Causal GQA attention of prompt rows over the KV cache on the bf16 matrix
+// cores, at the precision of f32.
+//
+// The reference computes scores, softmax and the weighted values of a prompt
+// row in f32 (paged_decode_scores_batched / decode_softmax_batched /
+// paged_decode_apply_batched, and the i8 pair of them over an int8 cache:
+// score = (q . code) * kscale * scale, context += (p * code) * vscale). Here
+// an f32 operand x is the exact sum of three bf16 numbers, x = x1 + x2 + x3
+// (8 + 8 + 8 significant bits, each the truncation of what the ones before it
+// leave), and a product of two such operands is the six partial products
+// x1y1, x1y2, x2y1, x2y2, x1y3, x3y1, accumulated in f32 by
+// v_mfma_f32_32x32x16_bf16. The three left out are below 2^-23 of the product,
+// the weight of one rounding in f32. Codes of the int8 cache are exact in one
+// bf16, so a product with them is three partial products.
+// f32 MFMA would take 64 cycles per 2048 multiply-adds, against 6 x 32 cycles
+// per 16384 here (3 x 32 with an int8 cache).
+//
+// One workgroup: QG x KS waves; wave (qg, ks) holds 32 query vectors (rows x
+// heads of one kv head's group) and walks the key tiles of 32 keys whose
+// index is ks mod KS, with its own running maximum, sum and context (online
+// softmax); at the end the KS parts are merged through LDS in a fixed order.
+// The tiles start at multiples of 32 positions and a masked tile leaves a
+// vector's state as it is, so a row's numbers do not depend on the rows it
+// shares a launch with: any chunking of a prompt gives the same bits.
+//
+// Scores are computed transposed (keys x queries): a lane then holds 16 keys
+// of one query, the softmax statistics need one exchange with lane ^ 32, and
+// the probabilities are already the B operand of (V^T x P^T) once V^T is
+// stored with its keys in the order the lanes hold them.
+//
+// K and V tiles go global -> registers -> (split) -> LDS; the loads of one go
+// out while the other is being multiplied.
+#include "bh_common.h"
+#include "bh_flash.h"
+
+namespace bh {
+namespace {
+
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+__device__ __forceinline__ uint32_t fbits(float f) { return __builtin_bit_cast(uint32_t, f); }
+__device__ __forceinline__ float bitsf(uint32_t u) { return __builtin_bit_cast(float, u); }
+// The upper halves of two floats: their truncations to bf16, packed.
+__device__ __forceinline__ uint32_t hi16x2(float lo, float hi) {
+    return __builtin_amdgcn_perm(fbits(hi), fbits(lo), 0x07060302u);
+}
+__device__ __forceinline__ float below_bf16(float x) { return x - bitsf(fbits(x) & 0xffff0000u); }
+
+// Eight floats as three bf16 fragments. (A non-finite operand leaves NaN in
+// the second part: its products are NaN.)
+__device__ __forceinline__ void split8(const float (&x)[8], v4i& a, v4i& b, v4i& c) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float x0 = x[2 * i], x1 = x[2 * i + 1];
+        a[i] = (int)hi16x2(x0, x1);
+        const float r0 = below_bf16(x0), r1 = below_bf16(x1);
+        b[i] = (int)hi16x2(r0, r1);
+        c[i] = (int)hi16x2(below_bf16(r0), below_bf16(r1));
+    }
+}
+__device__ __forceinline__ float code_f(uint32_t w, int e) { return (float)(int8_t)(uint8_t)(w >> (8 * e)); }
+
+__device__ __forceinline__ v16f mfma(v4i a, v4i b, v16f c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
+}
+
+template <bool KV8, int HD, int QG, int KS>
+struct FlashCfg {
+    static constexpr int NT = QG * KS * 64;
+    static constexpr int KEYS = 32 * KS;               // keys per step
+    static constexpr int PARTS = KV8 ? 1 : 3;          // bf16 parts of a cache element
+    static constexpr int TILE = 32 * HD * 2;           // bytes of one part of 32 keys
+    static constexpr int REGION = KS * PARTS * TILE;   // K, or V, of one step
+    static constexpr bool SEP = 2 * REGION <= 64 * 1024;  // K and V in LDS side by side
+    static constexpr int VOFF = SEP ? REGION : 0;
+    static constexpr int LDS = SEP ? 2 * REGION : REGION;
+    static constexpr int OREGS = HD / 2;               // context registers per lane
+    static constexpr int MERGE = (KS / 2) * QG * 64 * OREGS * 4;
+    static constexpr int NKC = KEYS * HD / 8 / NT;     // 8-element pieces of K per thread
+    static constexpr int VB = KEYS * HD / 32;          // 8-key x 4-d blocks of V
+    static constexpr int NVB = VB > NT ? VB / NT : 1;  // ... per thread (below VB, the first VB threads)
+    static constexpr int NR = NKC * 2 > NVB * 8 ? NKC * 2 : NVB * 8;
+    static_assert(NKC * NT * 8 == KEYS * HD && (VB <= NT || NVB * NT == VB), "whole pieces per thread");
+    static_assert(MERGE <= LDS, "the merge fits the tiles' LDS");
+};
+
+template <bool KV8, int HD, int QG, int KS>
+__global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p) {
+    using C = FlashCfg<KV8, HD, QG, KS>;
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[C::LDS];
+    __shared__ float sml[QG * KS][2][64];
+    __shared__ __attribute__((aligned(16))) float ksc[KV8 ? C::KEYS : 4], vsc[KV8 ? C::KEYS : 4];
+    __shared__ uint32_t btl[FLASH_MAX_TABLE];
+    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, col = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), qg = wave % QG, ks = wave / QG;
+    const int G = p.nh / p.nkv, RW = 32 / G;  // rows per wave
+    const int nqb = (p.rows_per_seq + RW * QG - 1) / (RW * QG);
+    // The blocks of the latest rows attend the most keys: they start first.
+    const int kh = blockIdx.x % p.nkv, bq = blockIdx.x / p.nkv;
+    const int b = bq % p.nseq, qb = nqb - 1 - bq / p.nseq;
+    const int i0 = qb * RW * QG, nrow = min(RW * QG, p.rows_per_seq - i0);
+    const int r0 = b * p.rows_per_seq + i0;
+    const size_t seq = p.seq[r0];
+    const int maxpos = (int)p.pos[r0 + nrow - 1];
+    const int niter = maxpos / C::KEYS + 1;
+    const bool paged = p.map.bs != 0;
+    if (paged) {
+        for (int i = tid; i <= maxpos / p.map.bs; i += C::NT) btl[i] = p.map.block(p.map.bt[seq * p.map.max_bt + i]);
+        __syncthreads();
+    }
+    auto slot_of = [&](int pos) -> size_t {
+        if (!paged) return seq * p.map.max_seq + pos;
+        const int blk = pos / p.map.bs;
+        return (size_t)btl[blk] * p.map.bs + (pos - blk * p.map.bs);
+    };
+
+    // This lane's query vector: row i of the block, head g of the group.
+    const int iw = qg * RW + (col < RW * G ? col / G : 0), g = col < RW * G ? col % G : 0;
+    const bool qlive = col < RW * G && iw < nrow;
+    float* qrow = p.q + (size_t)(r0 + min(iw, nrow - 1)) * p.hq + (size_t)(kh * G + g) * HD;
+    const int mypos = qlive ? (int)p.pos[r0 + iw] : -1;
+    const bool wlive = qg * RW < nrow;  // a wave without rows only helps to stage
+    const int wminpos = wlive ? (int)p.pos[r0 + qg * RW] : 0;
+    const int wmaxpos = wlive ? (int)p.pos[r0 + min(qg * RW + RW, nrow) - 1] : -1;
+    v4i qf[HD / 16][3];
+#pragma unroll
+    for (int s = 0; s < HD / 16; ++s) {
+        const float4 lo = *reinterpret_cast<const float4*>(qrow + 16 * s + 8 * half);
+        const float4 hi = *reinterpret_cast<const float4*>(qrow + 16 * s + 8 * half + 4);
+        const float x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+        split8(x, qf[s][0], qf[s][1], qf[s][2]);
+    }
+
+    // ---- staging
+    constexpr int CPK = HD / 8;  // 16-byte bf16 chunks per key
+    float4 rf[KV8 ? 1 : C::NR];  // K pieces, then V blocks, in flight
+    uint32_t r8[KV8 ? C::NR : 1];
+    float rsc = 0.0f;
+    auto kaddr = [&](int it, int u, int& key, int& c) -> size_t {
+        const int q = tid + u * C::NT;
+        key = q / CPK;
+        c = q % CPK;
+        return slot_of(min(it * C::KEYS + key, maxpos)) * p.hkv + (size_t)kh * HD + 8 * c;
+    };
+    auto load_scale = [&](int it, const float* sc) {
+        if constexpr (KV8) {
+            if (tid < C::KEYS) rsc = sc[slot_of(min(it * C::KEYS + tid, maxpos)) * p.nkv + kh];
+        }
+    };
+    auto load_k = [&](int it) {
+#pragma unroll
+        for (int u = 0; u < C::NKC; ++u) {
+            int key, c;
+            const size_t o = kaddr(it, u, key, c);
+            if constexpr (KV8) {
+                const uint2 v = *reinterpret_cast<const uint2*>(static_cast<const uint8_t*>(p.kc) + o);
+                r8[2 * u] = v.x;
+                r8[2 * u + 1] = v.y;
+            } else {
+                const float4* src = reinterpret_cast<const float4*>(static_cast<const float*>(p.kc) + o);
+                rf[2 * u] = src[0];
+                rf[2 * u + 1] = src[1];
+            }
+        }
+        load_scale(it, p.ks);
+    };
+    // LDS: K part t of tile w: [32 keys][HD] bf16, 16-byte chunk c of key r at
+    // c ^ (r & 15) (HD 64: c ^ (r >> 1 & 7)), so the 16 lanes of a fragment
+    // read on 16 rows hit 16 slots of a bank line.
+    auto kchunk = [&](int r, int c) -> int {
+        return r * (HD * 2) + ((HD == 128 ? c ^ (r & 15) : c ^ ((r >> 1) & 7)) << 4);
+    };
+    auto store_k = [&]() {
+#pragma unroll
+        for (int u = 0; u < C::NKC; ++u) {
+            const int q = tid + u * C::NT, key = q / CPK, c = q % CPK;
+            uint8_t* dst = lds + (key >> 5) * C::PARTS * C::TILE + kchunk(key & 31, c);
+            if constexpr (KV8) {
+                v4i w;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const uint32_t cw = r8[2 * u + (i >> 1)];
+                    w[i] = (int)hi16x2(code_f(cw, 2 * (i & 1)), code_f(cw, 2 * (i & 1) + 1));
+                }
+                *reinterpret_cast<v4i*>(dst) = w;
+            } else {
+                const float4 lo = rf[2 * u], hi = rf[2 * u + 1];
+                const float x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+                v4i w0, w1, w2;
+                split8(x, w0, w1, w2);
+                *reinterpret_cast<v4i*>(dst) = w0;
+                *reinterpret_cast<v4i*>(dst + C::TILE) = w1;
+                *reinterpret_cast<v4i*>(dst + 2 * C::TILE) = w2;
+            }
+        }
+        if constexpr (KV8)
+            if (tid < C::KEYS) ksc[tid] = rsc;
+    };
+    // A V block: 8 keys of one k-half of a 16-key step (the keys that half of
+    // the lanes holds of the scores: 4h..4h+3 and 8+4h..8+4h+3) x 4 d.
+    constexpr int DG = HD / 4;
+    auto vkey = [&](int oct, int j) -> int {  // octet of the step -> key of the step
+        const int in = oct & 3;
+        return 32 * (oct >> 2) + 16 * (in >> 1) + 4 * (in & 1) + (j < 4 ? j : 4 + j);
+    };
+    auto load_v = [&](int it) {
+#pragma unroll
+        for (int u = 0; u < C::NVB; ++u) {
+            const int q = tid + u * C::NT, oct = q / DG, dg = q % DG;
+            if (C::VB < C::NT && tid >= C::VB) break;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const size_t o = slot_of(min(it * C::KEYS + vkey(oct, j), maxpos)) * p.hkv + (size_t)kh * HD + 4 * dg;
+                if constexpr (KV8) r8[8 * u + j] = *reinterpret_cast<const uint32_t*>(static_cast<const uint8_t*>(p.vc) + o);
+                else rf[8 * u + j] = *reinterpret_cast<const float4*>(static_cast<const float*>(p.vc) + o);
+            }
+        }
+        load_scale(it, p.vs);
+    };
+    // LDS: V^T part t of tile w: lines of 256 bytes hold 4 d x 32 keys; the
+    // chunk of 8 keys (octet o) of d at slot (4 (d % 4) + o) ^ (line & 15) of
+    // line d / 4: neither the stores (16 lines, one d % 4 and o) nor the
+    // fragment reads (16 consecutive d, one o) meet in a bank.
+    auto vchunk = [&](int line, int d4, int o) -> int { return line * 256 + (((4 * d4 + o) ^ (line & 15)) << 4); };
+    auto store_v = [&]() {
+#pragma unroll
+        for (int u = 0; u < C::NVB; ++u) {
+            const int q = tid + u * C::NT, oct = q / DG, dg = q % DG;
+            if (C::VB < C::NT && tid >= C::VB) break;
+            uint8_t* base = lds + C::VOFF + (oct >> 2) * C::PARTS * C::TILE;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                uint8_t* dst = base + vchunk(dg, e, oct & 3);
+                float x[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    if constexpr (KV8) x[j] = code_f(r8[8 * u + j], e);
+                    else {
+                        const float4 v = rf[8 * u + j];
+                        x[j] = e == 0 ? v.x : e == 1 ? v.y : e == 2 ? v.z : v.w;
+                    }
+                }
+                if constexpr (KV8) {
+                    *reinterpret_cast<v4i*>(dst) = v4i{(int)hi16x2(x[0], x[1]), (int)hi16x2(x[2], x[3]),
+                                                       (int)hi16x2(x[4], x[5]), (int)hi16x2(x[6], x[7])};
+                } else {
+                    v4i w0, w1, w2;
+                    split8(x, w0, w1, w2);
+                    *reinterpret_cast<v4i*>(dst) = w0;
+                    *reinterpret_cast<v4i*>(dst + C::TILE) = w1;
+                    *reinterpret_cast<v4i*>(dst + 2 * C::TILE) = w2;
+                }
+            }
+        }
+        if constexpr (KV8)
+            if (tid < C::KEYS) vsc[tid] = rsc;
+    };
+    // Orders LDS only; the global loads in flight go on.
+    auto barrier = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    v16f o[HD / 32];
+#pragma unroll
+    for (int j = 0; j < HD / 32; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[j][e] = 0.0f;
+    float m = -INFINITY, l = 0.0f;  // l: this half's keys only
+
+    load_k(0);
+    for (int it = 0; it < niter; ++it) {
+        if constexpr (!C::SEP) barrier();  // the last step's V has been read
+        store_k();
+        load_v(it);
+        barrier();
+        const int j0 = it * C::KEYS + 32 * ks;
+        const bool live = j0 <= wmaxpos;  // wave-uniform
+        v16f s;
+        if (live) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) s[e] = 0.0f;
+            const uint8_t* kb = lds + ks * C::PARTS * C::TILE;
+#pragma unroll
+            for (int t = 0; t < HD / 16; ++t) {
+                const uint8_t* src = kb + kchunk(col, 2 * t + half);
+                const v4i k1 = *reinterpret_cast<const v4i*>(src);
+                if constexpr (KV8) {
+                    s = mfma(k1, qf[t][2], s);
+                    s = mfma(k1, qf[t][1], s);
+                    s = mfma(k1, qf[t][0], s);
+                } else {
+                    const v4i k2 = *reinterpret_cast<const v4i*>(src + C::TILE);
+                    const v4i k3 = *reinterpret_cast<const v4i*>(src + 2 * C::TILE);
+                    s = mfma(k3, qf[t][0], s);
+                    s = mfma(k1, qf[t][2], s);
+                    s = mfma(k2, qf[t][1], s);
+                    s = mfma(k2, qf[t][0], s);
+                    s = mfma(k1, qf[t][1], s);
+                    s = mfma(k1, qf[t][0], s);
+                }
+            }
+            // Register e: key 8 (e / 4) + 4 half + e % 4 of the tile.
+            if constexpr (KV8) {
+#pragma unroll
+                for (int e4 = 0; e4 < 4; ++e4) {
+                    const float4 k = *reinterpret_cast<const float4*>(ksc + 32 * ks + 8 * e4 + 4 * half);
+                    s[4 * e4] = s[4 * e4] * k.x;
+                    s[4 * e4 + 1] = s[4 * e4 + 1] * k.y;
+                    s[4 * e4 + 2] = s[4 * e4 + 2] * k.z;
+                    s[4 * e4 + 3] = s[4 * e4 + 3] * k.w;
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 16; ++e) s[e] = s[e] * p.scale;
+            if (j0 + 31 > wminpos) {
+                const int lim = mypos - j0 - 4 * half;  // keys of this half up to here are visible
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+                    if (8 * (e >> 2) + (e & 3) > lim) s[e] = -INFINITY;
+            }
+            float mx = s[0];
+#pragma unroll
+            for (int e = 1; e < 16; ++e) mx = fmaxf(mx, s[e]);
+            mx = fmaxf(mx, xor_lane<32>(mx));
+            const float mn = fmaxf(m, mx);
+            const float ref = mn == -INFINITY ? 0.0f : mn;  // no key seen yet: every weight is 0
+            if (__any(mn != m)) {
+                const float alpha = expf(m - ref);
+                l = l * alpha;
+#pragma unroll
+                for (int j = 0; j < HD / 32; ++j)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) o[j][e] = o[j][e] * alpha;
+                m = mn;
+            }
+            float sum = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                s[e] = expf(s[e] - ref);
+                sum = sum + s[e];
+            }
+            l = l + sum;
+        }
+        if constexpr (!C::SEP) barrier();  // every wave has read this step's K
+        store_v();
+        if (it + 1 < niter) load_k(it + 1);
+        barrier();
+        if (live) {
+            if constexpr (KV8) {
+#pragma unroll
+                for (int e4 = 0; e4 < 4; ++e4) {
+                    const float4 v = *reinterpret_cast<const float4*>(vsc + 32 * ks + 8 * e4 + 4 * half);
+                    s[4 * e4] = s[4 * e4] * v.x;
+                    s[4 * e4 + 1] = s[4 * e4 + 1] * v.y;
+                    s[4 * e4 + 2] = s[4 * e4 + 2] * v.z;
+                    s[4 * e4 + 3] = s[4 * e4 + 3] * v.w;
+                }
+            }
+            const uint8_t* vb = lds + C::VOFF + ks * C::PARTS * C::TILE;
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                float x[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) x[i] = s[8 * t + i];
+                v4i p1, p2, p3;
+                split8(x, p1, p2, p3);
+#pragma unroll
+                for (int j = 0; j < HD / 32; ++j) {
+                    const int d = 32 * j + col;
+                    const uint8_t* src = vb + vchunk(d >> 2, d & 3, 2 * t + half);
+                    const v4i v1 = *reinterpret_cast<const v4i*>(src);
+                    if constexpr (KV8) {
+                        o[j] = mfma(v1, p3, o[j]);
+                        o[j] = mfma(v1, p2, o[j]);
+                        o[j] = mfma(v1, p1, o[j]);
+                    } else {
+                        const v4i v2 = *reinterpret_cast<const v4i*>(src + C::TILE);
+                        const v4i v3 = *reinterpret_cast<const v4i*>(src + 2 * C::TILE);
+                        o[j] = mfma(v3, p1, o[j]);
+                        o[j] = mfma(v1, p3, o[j]);
+                        o[j] = mfma(v2, p2, o[j]);
+                        o[j] = mfma(v2, p1, o[j]);
+                        o[j] = mfma(v1, p2, o[j]);
+                        o[j] = mfma(v1, p1, o[j]);
+                    }
+                }
+            }
+        }
+    }
+
+    // Merge the KS parts: the upper half of the waves hands its state to the
+    // lower half, until one wave per query group is left.
+#pragma unroll
+    for (int w = KS / 2; w >= 1; w /= 2) {
+        barrier();
+        float4* om = reinterpret_cast<float4*>(lds) + (size_t)((ks % w) * QG + qg) * 64 * (HD / 8) + lane;
+        if (ks >= w && ks < 2 * w) {
+#pragma unroll
+            for (int j = 0; j < HD / 32; ++j)
+#pragma unroll
+                for (int e4 = 0; e4 < 4; ++e4)
+                    om[(4 * j + e4) * 64] = make_float4(o[j][4 * e4], o[j][4 * e4 + 1], o[j][4 * e4 + 2], o[j][4 * e4 + 3]);
+            sml[(ks % w) * QG + qg][0][lane] = m;
+            sml[(ks % w) * QG + qg][1][lane] = l;
+        }
+        barrier();
+        if (ks < w) {
+            const float m2 = sml[(ks % w) * QG + qg][0][lane], l2 = sml[(ks % w) * QG + qg][1][lane];
+            const float mn = fmaxf(m, m2), ref = mn == -INFINITY ? 0.0f : mn;
+            const float a1 = expf(m - ref), a2 = expf(m2 - ref);
+            m = mn;
+            l = l * a1 + l2 * a2;
+#pragma unroll
+            for (int j = 0; j < HD / 32; ++j)
+#pragma unroll
+                for (int e4 = 0; e4 < 4; ++e4) {
+                    const float4 v = om[(4 * j + e4) * 64];
+                    o[j][4 * e4] = o[j][4 * e4] * a1 + v.x * a2;
+                    o[j][4 * e4 + 1] = o[j][4 * e4 + 1] * a1 + v.y * a2;
+                    o[j][4 * e4 + 2] = o[j][4 * e4 + 2] * a1 + v.z * a2;
+                    o[j][4 * e4 + 3] = o[j][4 * e4 + 3] * a1 + v.w * a2;
+                }
+        }
+    }
+    if (ks == 0) {
+        const float inv = 1.0f / (l + xor_lane<32>(l));
+        if (qlive) {
+#pragma unroll
+            for (int j = 0; j < HD / 32; ++j)
+#pragma unroll
+                for (int e4 = 0; e4 < 4; ++e4)
+                    *reinterpret_cast<float4*>(qrow + 32 * j + 8 * e4 + 4 * half) =
+                        make_float4(o[j][4 * e4] * inv, o[j][4 * e4 + 1] * inv, o[j][4 * e4 + 2] * inv,
+                                    o[j][4 * e4 + 3] * inv);
+        }
+    }
+}
+
+template <bool KV8, int HD, int QG, int KS>
+hipError_t go(hipStream_t s, const FlashArgs& a) {
+    const int rb = 32 / (a.nh / a.nkv) * QG;
+    const unsigned grid = (unsigned)((a.rows_per_seq + rb - 1) / rb * a.nseq * a.nkv);
+    flash_prefill_kernel<KV8, HD, QG, KS><<<grid, QG * KS * 64, 0, s>>>(a);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_flash_prefill(hipStream_t s, const FlashArgs& a, int hd, bool kv8) {
+    if (a.rows_per_seq <= 0 || a.nseq <= 0) return hipSuccess;
+    if (hd == 128) return kv8 ? go<true, 128, 2, 4>(s, a) : go<false, 128, 2, 4>(s, a);
+    return kv8 ? go<true, 64, 2, 4>(s, a) : go<false, 64, 2, 4>(s, a);
+}
+
+}  // namespace bh

@@ -44,6 +44,7 @@
 #include "../../include/brain_hip.h"
 #include "bh_attn.h"
 #include "bh_common.h"
+#include "bh_flash.h"
 #include "bh_st.h"
 
 namespace bh {
@@ -218,27 +219,6 @@ __global__ __launch_bounds__(NT) void swiglu_quant_kernel(const float* gu, int f
     }
     quant_row<G, NT, false>(h, d4, red, sx + r, xq + (size_t)r * xq_words);
 }
-
-// Where position `pos` of sequence `seq` lives in a layer's cache: the token
-// slot whose K (V) row is [slot][hkv] and whose KV8 scales are [slot][nkv].
-// Contiguous slabs (bs == 0): slot = seq * max_seq + pos. Paged pool
-// (crates/qwen3/src/serve.rs:349-356, the layout of
-// paged_kv_append_i8_clipped_batched.wgsl:46-77): slot = block * bs + pos % bs
-// with block = bt[seq * max_bt + pos / bs]; bs is a multiple of the attention
-// chunk, so a chunk of keys lies inside one block. A table entry outside the
-// pool (an unallocated block) maps to block 0: only chunks past a row's
-// position read it (their reads are issued before the position is known and
-// never used), and the host refuses to run a row whose used blocks are not
-// allocated.
-struct KvMap {
-    const uint32_t* bt;  // [max_batch][max_bt] physical blocks (paged)
-    int max_bt, bs, nblk, max_seq;
-    __device__ __forceinline__ size_t slot(size_t seq, int pos) const {
-        if (bs == 0) return seq * max_seq + pos;
-        const uint32_t blk = bt[seq * max_bt + pos / bs];
-        return (size_t)(blk < (uint32_t)nblk ? blk : 0u) * bs + pos % bs;
-    }
-};
 
 struct RopeArgs {
     const float* qkv;  // [rows, hq + 2 hkv]
@@ -766,187 +746,6 @@ __global__ __launch_bounds__(RT) void attn_split_kernel(AttnArgs p) {
     }
 }
 
-// Prefill attention over query blocks: one workgroup per (sequence, block
-// of QB consecutive rows of that sequence, chunk of 32 keys; kv head), QB*G =
-// 32 query vectors (row i, head g). The chunk's K and V go through LDS once
-// for all 32 queries (attn_split_kernel reloads them per row). Like the split
-// kernel it writes, per (row, head, chunk), the chunk's softmax statistics
-// (max m, sum l) and its unnormalized weighted sum of V; attn_combine_quant
-// merges the chunks. A query's numbers depend only on its own row and the
-// chunk, not on the rows it shares a block with, so any chunking of the
-// prompt gives the same bits.
-constexpr int PQ = 32;  // query vectors per prefill workgroup
-template <bool KV8, int HD>
-__global__ __launch_bounds__(RT) void attn_prefill_kernel(AttnArgs p, int rows_per_seq) {
-    extern __shared__ __attribute__((aligned(16))) float pf_dyn[];
-    constexpr int hd = HD, hd4 = hd >> 2, ks = hd + 4;  // K rows padded for the LDS banks
-    constexpr int NP = PQ * hd / 4 / RT;                // float4 pieces per thread (Q, K, V alike)
-    static_assert(NP >= 1 && NP * RT * 4 == PQ * hd && KCH * hd4 == NP * RT, "whole pieces per thread");
-    constexpr int ow = hd >> 3;                         // head_dim slice per thread in P.V
-    const int G = p.nh / p.nkv, QB = PQ / G;
-    const int nqb = (rows_per_seq + QB - 1) / QB;
-    const int sp = blockIdx.x % p.splits, bq = blockIdx.x / p.splits;
-    const int b = bq / nqb, qb = bq - b * nqb, kh = blockIdx.y, tid = threadIdx.x;
-    const int i0 = qb * QB, nrow = min(QB, rows_per_seq - i0);
-    const int r0 = b * rows_per_seq + i0;  // first row of the block
-    const int j0 = sp * KCH;
-    // Rows are consecutive positions: the last row holds the largest.
-    const int maxpos = (int)p.pos[r0 + nrow - 1];
-    if (j0 > maxpos) return;
-    const int nk = min(KCH, maxpos + 1 - j0);
-    float* Qs = pf_dyn;         // [PQ][hd]
-    float* Ks = Qs + PQ * hd;   // [32][hd + 4]
-    float* Vs = Ks + KCH * ks;  // [32][hd]
-    __shared__ float Ps[PQ][KCH + 1];
-    __shared__ float mls[PQ][2];
-    __shared__ int posq[PQ];
-    __shared__ float ksc[KCH], vsc[KCH];
-    const size_t seq = p.seq[r0];
-    const size_t tok0 = p.ro.map.slot(seq, j0);  // cache slot of this chunk's first key
-    const size_t base = tok0 * p.hkv + (size_t)kh * hd;
-    // Every global read is issued before the first use.
-    float4 qv[NP], kf[KV8 ? 1 : NP], vf[KV8 ? 1 : NP];
-    uint32_t k8[KV8 ? NP : 1], v8[KV8 ? NP : 1];
-#pragma unroll
-    for (int u = 0; u < NP; ++u) {
-        const int idx = tid + u * RT, q = idx / hd4, c = (idx - q * hd4) * 4, i = q / G, g = q - i * G;
-        qv[u] = i < nrow ? *reinterpret_cast<const float4*>(p.q + (size_t)(r0 + i) * p.hq + (size_t)(kh * G + g) * hd + c)
-                         : make_float4(0.f, 0.f, 0.f, 0.f);
-        const int k = idx / hd4;  // the same piece index over the K / V chunk
-        const bool live = k < nk;
-        const size_t o = base + (size_t)k * p.hkv + c;
-        if constexpr (KV8) {
-            k8[u] = live ? *reinterpret_cast<const uint32_t*>(static_cast<const uint8_t*>(p.kc) + o) : 0u;
-            v8[u] = live ? *reinterpret_cast<const uint32_t*>(static_cast<const uint8_t*>(p.vc) + o) : 0u;
-        } else {
-            kf[u] = live ? *reinterpret_cast<const float4*>(static_cast<const float*>(p.kc) + o) : make_float4(0.f, 0.f, 0.f, 0.f);
-            vf[u] = live ? *reinterpret_cast<const float4*>(static_cast<const float*>(p.vc) + o) : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-    }
-    float scl = 0.0f;
-    if constexpr (KV8) {
-        const int k = tid < KCH ? tid : tid - KCH;
-        if (tid < 2 * KCH && k < nk) scl = (tid < KCH ? p.ks : p.vs)[(tok0 + k) * p.nkv + kh];
-    }
-    if (tid < PQ) {
-        const int i = tid / G;
-        posq[tid] = i < nrow ? (int)p.pos[r0 + i] : -1;
-    }
-#pragma unroll
-    for (int u = 0; u < NP; ++u) {
-        const int idx = tid + u * RT, q = idx / hd4, c = (idx - q * hd4) * 4;
-        *reinterpret_cast<float4*>(Qs + q * hd + c) = qv[u];
-        if constexpr (KV8) {
-            *reinterpret_cast<float4*>(Ks + q * ks + c) = i8x4(k8[u]);
-            *reinterpret_cast<float4*>(Vs + q * hd + c) = i8x4(v8[u]);
-        } else {
-            *reinterpret_cast<float4*>(Ks + q * ks + c) = kf[u];
-            *reinterpret_cast<float4*>(Vs + q * hd + c) = vf[u];
-        }
-    }
-    if constexpr (KV8) {
-        if (tid < KCH) ksc[tid] = scl;
-        else if (tid < 2 * KCH) vsc[tid - KCH] = scl;
-    }
-    __syncthreads();
-    // Scores: thread -> queries 2*(t>>4)+{0,1} x keys 2*(t&15)+{0,1}, each dot
-    // product in head_dim order, then (KV8: x kscale) x 1/sqrt(hd).
-    {
-        const int q0 = 2 * (tid >> 4), k0 = 2 * (tid & 15);
-        float s00 = 0.f, s01 = 0.f, s10 = 0.f, s11 = 0.f;
-        const float* qa = Qs + q0 * hd;
-        const float* qb2 = qa + hd;
-        const float* ka = Ks + k0 * ks;
-        const float* kb = ka + ks;
-#pragma unroll 8
-        for (int c = 0; c < hd; c += 4) {
-            const float4 a0 = *reinterpret_cast<const float4*>(qa + c), a1 = *reinterpret_cast<const float4*>(qb2 + c);
-            const float4 b0 = *reinterpret_cast<const float4*>(ka + c), b1 = *reinterpret_cast<const float4*>(kb + c);
-            s00 += a0.x * b0.x + a0.y * b0.y + a0.z * b0.z + a0.w * b0.w;
-            s01 += a0.x * b1.x + a0.y * b1.y + a0.z * b1.z + a0.w * b1.w;
-            s10 += a1.x * b0.x + a1.y * b0.y + a1.z * b0.z + a1.w * b0.w;
-            s11 += a1.x * b1.x + a1.y * b1.y + a1.z * b1.z + a1.w * b1.w;
-        }
-        const float sv[2][2] = {{s00, s01}, {s10, s11}};
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int c = 0; c < 2; ++c) {
-                const int q = q0 + a, k = k0 + c;
-                float v = sv[a][c];
-                if (KV8) v = v * ksc[k];
-                v = v * p.scale;
-                const bool live = k < nk && posq[q] >= 0 && j0 + k <= posq[q];
-                Ps[q][k] = live ? v : -INFINITY;
-            }
-    }
-    __syncthreads();
-    // The chunk's statistics: 8 lanes per query, 4 keys each; max and sum
-    // over the 8 lanes by xor shuffles (a fixed order per query).
-    {
-        const int q = tid >> 3, k4 = (tid & 7) * 4;
-        float sv[4];
-        float mx = -INFINITY;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            sv[c] = Ps[q][k4 + c];
-            mx = fmaxf(mx, sv[c]);
-        }
-        mx = fmaxf(mx, xor_lane<1>(mx));
-        mx = fmaxf(mx, xor_lane<2>(mx));
-        mx = fmaxf(mx, xor_lane<4>(mx));
-        float sum = 0.0f;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            sv[c] = sv[c] == -INFINITY ? 0.0f : expf(sv[c] - mx);
-            sum += sv[c];
-        }
-        sum += xor_lane<1>(sum);
-        sum += xor_lane<2>(sum);
-        sum += xor_lane<4>(sum);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) Ps[q][k4 + c] = sv[c];
-        if ((tid & 7) == 0) {
-            mls[q][0] = mx;
-            mls[q][1] = sum;
-        }
-    }
-    __syncthreads();
-    // o = sum_k p_k v_k over the chunk's keys in order.
-    const int oq = tid >> 3, od = (tid & 7) * ow;
-    const int i = oq / G, g = oq - i * G;
-    if (i >= nrow || j0 > posq[oq]) return;  // no key of this chunk is visible to the query
-    float O[ow];
-#pragma unroll
-    for (int u = 0; u < ow; ++u) O[u] = 0.0f;
-#pragma unroll 4
-    for (int k = 0; k < nk; ++k) {
-        const float pk = Ps[oq][k];
-        float vk[ow];
-#pragma unroll
-        for (int u = 0; u < ow; u += 4) {
-            const float4 x = *reinterpret_cast<const float4*>(Vs + k * hd + od + u);
-            vk[u] = x.x; vk[u + 1] = x.y; vk[u + 2] = x.z; vk[u + 3] = x.w;
-        }
-        if constexpr (KV8) {
-            const float vs = vsc[k];
-#pragma unroll
-            for (int u = 0; u < ow; ++u) O[u] += pk * vk[u] * vs;
-        } else {
-#pragma unroll
-            for (int u = 0; u < ow; ++u) O[u] += pk * vk[u];
-        }
-    }
-    const size_t slot = ((size_t)(r0 + i) * p.nh + kh * G + g) * p.splits + sp;
-#pragma unroll
-    for (int u = 0; u < ow; u += 4)
-        *reinterpret_cast<float4*>(p.part_o + slot * hd + od + u) = make_float4(O[u], O[u + 1], O[u + 2], O[u + 3]);
-    if ((tid & 7) == 0) {
-        p.part_ml[2 * slot] = mls[oq][0];
-        p.part_ml[2 * slot + 1] = mls[oq][1];
-    }
-}
-
 // Merge the key chunks of every head of row r: M = max m_s,
 // L = sum l_s e^(m_s - M), ctx = sum o_s e^(m_s - M) / L; then quantize the
 // whole context row for the output projection (quant_pack semantics).
@@ -1205,6 +1004,7 @@ struct bh_qwen3 {
     float *res = nullptr, *res2 = nullptr, *qkv = nullptr, *q = nullptr, *proj = nullptr, *gu = nullptr;
     float *part_o = nullptr, *part_ml = nullptr;  // attention chunk partials
     uint32_t max_splits = 0;
+    bool flash = false;  // prompt attention on launch_flash_prefill (else attn_split + merge)
     const uint32_t* cur_pos = nullptr;
     float *sx = nullptr, *logits = nullptr, *tmpw = nullptr, *am_v = nullptr;
     uint32_t *xq = nullptr, *am_i = nullptr, *am_n = nullptr;  // xq: every producer writes rows of width/4 words
@@ -1376,8 +1176,8 @@ static bool am_separate() {
 // `splits`: key chunks of KCH covering the longest row of this launch (the
 // workspace stride; chunks past a row's position exit immediately).
 // `rows_per_seq` > 0: the rows are whole runs of consecutive positions, one
-// run of that many rows per sequence (a prefill chunk), which the
-// query-block attention kernel needs.
+// run of that many rows per sequence (a prefill chunk), which the flash
+// kernel needs.
 int run_rows(bh_qwen3* e, int rows, const uint32_t* tok, const uint32_t* pos, const uint32_t* seq, int n_out,
              const int* out_map, bool decode, int splits, int rows_per_seq = 0) {
     e->cur_pos = pos;
@@ -1387,11 +1187,8 @@ int run_rows(bh_qwen3* e, int rows, const uint32_t* tok, const uint32_t* pos, co
     float* nxt = e->res2;
     const int nh = (int)c.n_heads, nkv = (int)c.n_kv_heads;
     const float scale = 1.0f / sqrtf((float)hd);
-    // Query-block prefill attention: whole per-sequence runs, 32 query vectors
-    // a workgroup (G divides 32), head_dim 64 or 128 (the kernel is built for
-    // those; its LDS image stays within 64 KB).
-    const bool qblock = !decode && rows_per_seq > 0 && rows % rows_per_seq == 0 && PQ % (nh / nkv) == 0 &&
-                        (hd == 64 || hd == 128);
+    // Prompt rows: whole runs of consecutive positions, one per sequence.
+    const bool flash = !decode && rows_per_seq > 0 && rows % rows_per_seq == 0 && e->flash;
     for (uint32_t l = 0; l < c.n_layers; ++l) {
         const bh_qwen3::Layer& Ly = e->L[l];
         void* kc = static_cast<uint8_t*>(e->kc) + l * e->layer_kv * e->kv_elem;
@@ -1455,17 +1252,10 @@ int run_rows(bh_qwen3* e, int rows, const uint32_t* tok, const uint32_t* pos, co
             if (c.kv_int8) qk_rope_append_kernel<true><<<dim3(rows, nh + 2 * nkv), 64, 0, e->stream>>>(ra);
             else qk_rope_append_kernel<false><<<dim3(rows, nh + 2 * nkv), 64, 0, e->stream>>>(ra);
             BH_HIP(hipGetLastError(), "qk_rope_append launch");
-            if (qblock) {
-                const int nqb = (rows_per_seq + PQ / (nh / nkv) - 1) / (PQ / (nh / nkv));
-                const dim3 pgrid(rows / rows_per_seq * nqb * splits, nkv);
-                const size_t plds = ((size_t)PQ * hd + (size_t)KCH * (hd + 4) + (size_t)KCH * hd) * 4;
-                if (hd == 128) {
-                    if (c.kv_int8) attn_prefill_kernel<true, 128><<<pgrid, RT, plds, e->stream>>>(aa, rows_per_seq);
-                    else attn_prefill_kernel<false, 128><<<pgrid, RT, plds, e->stream>>>(aa, rows_per_seq);
-                } else {
-                    if (c.kv_int8) attn_prefill_kernel<true, 64><<<pgrid, RT, plds, e->stream>>>(aa, rows_per_seq);
-                    else attn_prefill_kernel<false, 64><<<pgrid, RT, plds, e->stream>>>(aa, rows_per_seq);
-                }
+            if (flash) {
+                const FlashArgs fa{e->q, kc, vc, ksl, vsl, pos, seq, nh, nkv, (int)e->hq, (int)e->hkv, rows_per_seq,
+                                   rows / rows_per_seq, scale, ra.map};
+                BH_HIP(launch_flash_prefill(e->stream, fa, hd, c.kv_int8 != 0), "attention launch");
             } else {
                 if (c.kv_int8) attn_split_kernel<true><<<agrid, RT, alds_pre, e->stream>>>(aa);
                 else attn_split_kernel<false><<<agrid, RT, alds_pre, e->stream>>>(aa);
@@ -1478,13 +1268,14 @@ int run_rows(bh_qwen3* e, int rows, const uint32_t* tok, const uint32_t* pos, co
         // thread with the loads issued before the position read, which costs
         // less than a launch. With more rows each workgroup merges them one
         // after another (measured slower from 2 rows: batch 4 1.19 -> 1.43 ms).
-        if (fuse && rows == 1 && fused_ok(rows, (int)e->hq, d, 1) && e->hq <= 2048) {
+        if (!flash && fuse && rows == 1 && fused_ok(rows, (int)e->hq, d, 1) && e->hq <= 2048) {
             // The merge of the chunks inside the output projection's prologue.
             BH_HIP(launch_gemv_i8_merge(e->stream, e->part_o, e->part_ml, e->cur_pos, nh, hd, splits, Ly.wo, Ly.so,
                                         e->proj, rows, (int)e->hq / 4, d),
                    "fused merge + output projection launch");
         } else {
-            BH_TRY(launch_combine_quant(e, rows, splits));
+            if (flash) BH_HIP(launch_quantize_rows(e->stream, e->q, rows, (int)e->hq, e->sx, e->xq), "context quantization");
+            else BH_TRY(launch_combine_quant(e, rows, splits));
             BH_TRY(launch_linear(e, Ly.wo, Ly.so, e->proj, rows, (int)e->hq, d));
         }
         if (fuse) {
@@ -1745,6 +1536,8 @@ int bh_qwen3_create(const bh_qwen3_config* cfg, uint32_t max_batch, uint32_t max
     e->tmpw_floats = std::max<uint64_t>(std::max<uint64_t>((uint64_t)e->W * d, 2 * ff * d), d * std::max<uint64_t>(hq, ff));
     if (!c.tie_embeddings) e->tmpw_floats = std::max<uint64_t>(e->tmpw_floats, (uint64_t)c.vocab * d);
     const uint64_t R = max_rows;
+    e->flash = flash_ok((int)c.head_dim, (int)c.n_heads, (int)c.n_kv_heads, (int)e->kv_max_bt);
+    const uint64_t PR = e->flash ? max_batch : R;  // rows of chunk partials: decode rows, or prompt rows too
     if ((rc = dalloc(e, &e->emb, (uint64_t)c.vocab * d)) || (rc = dalloc(e, &e->norm, d)) ||
         (rc = dalloc(e, &e->head, (uint64_t)c.vocab * d / 4)) || (rc = dalloc(e, &e->shead, c.vocab)) ||
         (rc = dalloc(e, (uint8_t**)&e->kc, e->layer_kv * c.n_layers * e->kv_elem)) ||
@@ -1756,7 +1549,8 @@ int bh_qwen3_create(const bh_qwen3_config* cfg, uint32_t max_batch, uint32_t max
         (rc = dalloc(e, &e->vclip, (uint64_t)c.n_layers * c.n_kv_heads)) ||
         (rc = dalloc(e, &e->rope_cs, (uint64_t)max_seq * (c.head_dim / 2))) ||
         (rc = dalloc(e, &e->res, R * d)) || (rc = dalloc(e, &e->res2, R * d)) || (rc = dalloc(e, &e->qkv, R * e->W)) || (rc = dalloc(e, &e->q, R * hq)) ||
-        (rc = dalloc(e, &e->part_o, R * c.n_heads * e->max_splits * c.head_dim)) || (rc = dalloc(e, &e->part_ml, R * c.n_heads * e->max_splits * 2)) || (rc = dalloc(e, &e->proj, R * d)) || (rc = dalloc(e, &e->gu, R * 2 * ff)) ||
+        (rc = dalloc(e, &e->part_o, PR * c.n_heads * e->max_splits * c.head_dim)) ||
+        (rc = dalloc(e, &e->part_ml, PR * c.n_heads * e->max_splits * 2)) || (rc = dalloc(e, &e->proj, R * d)) || (rc = dalloc(e, &e->gu, R * 2 * ff)) ||
         (rc = dalloc(e, &e->sx, R)) || (rc = dalloc(e, &e->xq, R * e->xq_words)) ||
         (rc = dalloc(e, &e->logits, (uint64_t)max_batch * c.vocab)) || (rc = dalloc(e, &e->tmpw, e->tmpw_floats)) ||
         (rc = dalloc(e, &e->am_v, (uint64_t)max_batch * AM_PARTS)) || (rc = dalloc(e, &e->am_i, (uint64_t)max_batch * AM_PARTS)) ||
