@@ -19,10 +19,10 @@ namespace bh {
 struct KvMap {
     const uint32_t* bt;  // [max_batch][max_bt] physical blocks (paged)
     int max_bt, bs, nblk, max_seq;
-    __device__ __forceinline__ uint32_t block(uint32_t entry) const { return entry < (uint32_t)nblk ? entry : 0u; }
     __device__ __forceinline__ size_t slot(size_t seq, int pos) const {
         if (bs == 0) return seq * max_seq + pos;
-        return (size_t)block(bt[seq * max_bt + pos / bs]) * bs + pos % bs;
+        const uint32_t blk = bt[seq * max_bt + pos / bs];
+        return (size_t)(blk < (uint32_t)nblk ? blk : 0u) * bs + pos % bs;
     }
 };
 
@@ -41,11 +41,11 @@ struct FlashArgs {
 };
 
 constexpr int FLASH_MAX_GROUP = 8;       // query heads per kv head
-constexpr int FLASH_MAX_TABLE = 2048;    // block-table entries of one sequence
+constexpr int FLASH_MAX_SEQ = 65536;     // positions of one sequence
 
 // Whether launch_flash_prefill is built for this geometry.
-inline bool flash_ok(int hd, int nh, int nkv, int max_bt) {
-    return (hd == 64 || hd == 128) && nh / nkv <= FLASH_MAX_GROUP && max_bt <= FLASH_MAX_TABLE;
+inline bool flash_ok(int hd, int nh, int nkv, int max_seq) {
+    return (hd == 64 || hd == 128) && nh / nkv <= FLASH_MAX_GROUP && max_seq <= FLASH_MAX_SEQ;
 }
 hipError_t launch_flash_prefill(hipStream_t s, const FlashArgs& a, int hd, bool kv8);
 

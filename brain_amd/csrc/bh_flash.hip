@@ -30,6 +30,22 @@
 //
 // K and V tiles go global -> registers -> (split) -> LDS; the loads of one go
 // out while the other is being multiplied.
+//
+// Measured, 16 query heads over 8 kv heads of 128, one 2000-token prompt /
+// eight of 250: int8 cache 80 / 31 us, f32 cache 175 / 39 us. (The kernel
+// before it, f32 products on the vector units with 32-key partial sums through
+// memory, and its merge: 964 + 138 us for the 2000 tokens, int8.) At 2000
+// tokens the matrix cores are busy 30% of the time and vector instructions
+// issue in 48%: the conversion of the tiles to bf16 and the softmax bound it.
+// Waves: 2 x 4 for the int8 cache; for the f32 cache, whose split tiles take
+// three times the LDS, 2 x 2 with two workgroups per CU measured 175 / 39 us
+// against 164 / 51 us at 2 x 4, and 12 against 17 us at 64 tokens. KS is part
+// of the result's summation order, so it is one per cache type and not chosen
+// by length. Against 64-bit attention, one 2000-token prompt of normal q, k, v:
+// 1.6e-7 (f32 cache) and 3.0e-7 (int8) in the 2-norm; the f32 kernel 2.2e-7
+// and 3.3e-7.
+#include <type_traits>
+
 #include "bh_common.h"
 #include "bh_flash.h"
 
@@ -59,6 +75,19 @@ __device__ __forceinline__ void split8(const float (&x)[8], v4i& a, v4i& b, v4i&
         c[i] = (int)hi16x2(below_bf16(r0), below_bf16(r1));
     }
 }
+// Softmax in base 2: a weight is exp2(fma(score, c, -m)) with
+// c = scale * log2(e) and m the reference of the same base, one rounding at
+// the size of the difference (the scaled score itself is never rounded).
+// The reference is not the running maximum but within SLACK of it: it moves
+// only when a key's score is more than SLACK above it, which spares most
+// tiles the rescaling of the context; weights are then up to 2^SLACK, with the
+// same relative precision. Each row decides for itself.
+constexpr float SLACK = 8.0f;
+// The score of a masked key, and a row's reference before its first key:
+// finite, so that their differences are, and far enough apart that a masked
+// key (times c >= 1/16) weighs 0 against either.
+constexpr float MASKED = -1.0e38f, NO_REF = -1.0e34f;
+
 __device__ __forceinline__ float code_f(uint32_t w, int e) { return (float)(int8_t)(uint8_t)(w >> (8 * e)); }
 
 __device__ __forceinline__ v16f mfma(v4i a, v4i b, v16f c) {
@@ -89,9 +118,13 @@ template <bool KV8, int HD, int QG, int KS>
 __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p) {
     using C = FlashCfg<KV8, HD, QG, KS>;
     __shared__ __attribute__((aligned(1024))) uint8_t lds[C::LDS];
+    // The third parts of the queries (one use per key tile) live in LDS: 32
+    // registers fewer at head_dim 128, which is what keeps the kernel from
+    // spilling at two waves per SIMD.
+    __shared__ __attribute__((aligned(1024))) uint8_t q3[QG * C::TILE];
     __shared__ float sml[QG * KS][2][64];
     __shared__ __attribute__((aligned(16))) float ksc[KV8 ? C::KEYS : 4], vsc[KV8 ? C::KEYS : 4];
-    __shared__ uint32_t btl[FLASH_MAX_TABLE];
+    __shared__ uint32_t tslot[FLASH_MAX_SEQ / 32];
     const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, col = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), qg = wave % QG, ks = wave / QG;
     const int G = p.nh / p.nkv, RW = 32 / G;  // rows per wave
@@ -104,16 +137,8 @@ __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p)
     const size_t seq = p.seq[r0];
     const int maxpos = (int)p.pos[r0 + nrow - 1];
     const int niter = maxpos / C::KEYS + 1;
-    const bool paged = p.map.bs != 0;
-    if (paged) {
-        for (int i = tid; i <= maxpos / p.map.bs; i += C::NT) btl[i] = p.map.block(p.map.bt[seq * p.map.max_bt + i]);
-        __syncthreads();
-    }
-    auto slot_of = [&](int pos) -> size_t {
-        if (!paged) return seq * p.map.max_seq + pos;
-        const int blk = pos / p.map.bs;
-        return (size_t)btl[blk] * p.map.bs + (pos - blk * p.map.bs);
-    };
+    // First slot of every 32-key tile (a tile lies inside one block).
+    for (int i = tid; i <= maxpos >> 5; i += C::NT) tslot[i] = (uint32_t)p.map.slot(seq, 32 * i);
 
     // This lane's query vector: row i of the block, head g of the group.
     const int iw = qg * RW + (col < RW * G ? col / G : 0), g = col < RW * G ? col % G : 0;
@@ -123,53 +148,73 @@ __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p)
     const bool wlive = qg * RW < nrow;  // a wave without rows only helps to stage
     const int wminpos = wlive ? (int)p.pos[r0 + qg * RW] : 0;
     const int wmaxpos = wlive ? (int)p.pos[r0 + min(qg * RW + RW, nrow) - 1] : -1;
-    v4i qf[HD / 16][3];
+    // LDS image of 32 rows of HD bf16 (a tile of K, or a wave's q3): 16-byte
+    // chunk c of row r at c ^ (r & 15) (HD 64: c ^ (r >> 1 & 7)), so the 16
+    // lanes of a fragment read on 16 rows hit 16 slots of a bank line.
+    auto kchunk = [&](int r, int c) -> int {
+        return r * (HD * 2) + ((HD == 128 ? c ^ (r & 15) : c ^ ((r >> 1) & 7)) << 4);
+    };
+    const uint8_t* q3w = q3 + qg * C::TILE;
+    v4i qf[HD / 16][2];
 #pragma unroll
     for (int s = 0; s < HD / 16; ++s) {
         const float4 lo = *reinterpret_cast<const float4*>(qrow + 16 * s + 8 * half);
         const float4 hi = *reinterpret_cast<const float4*>(qrow + 16 * s + 8 * half + 4);
         const float x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-        split8(x, qf[s][0], qf[s][1], qf[s][2]);
+        v4i third;
+        split8(x, qf[s][0], qf[s][1], third);
+        if (ks == 0) *reinterpret_cast<v4i*>(q3 + qg * C::TILE + kchunk(col, 2 * s + half)) = third;
     }
+    __syncthreads();  // tslot, q3
 
     // ---- staging
     constexpr int CPK = HD / 8;  // 16-byte bf16 chunks per key
     float4 rf[KV8 ? 1 : C::NR];  // K pieces, then V blocks, in flight
     uint32_t r8[KV8 ? C::NR : 1];
     float rsc = 0.0f;
-    auto kaddr = [&](int it, int u, int& key, int& c) -> size_t {
-        const int q = tid + u * C::NT;
-        key = q / CPK;
-        c = q % CPK;
-        return slot_of(min(it * C::KEYS + key, maxpos)) * p.hkv + (size_t)kh * HD + 8 * c;
+    // A tile's first cache row of this kv head, as a uniform element offset,
+    // and its last visible key. Keys past that repeat it: their weights are
+    // zero, and what they multiply is a value that is visible.
+    struct TileAt {
+        size_t base;
+        int last;
     };
+    auto tile_at = [&](int it, int w) -> TileAt {  // w: uniform
+        const int t0 = min(it * KS + w, maxpos >> 5);
+        const uint32_t slot = (uint32_t)__builtin_amdgcn_readfirstlane((int)tslot[t0]);
+        return {(size_t)slot * (uint32_t)p.hkv + (uint32_t)(kh * HD), min(maxpos - 32 * t0, 31)};
+    };
+    using Elem = std::conditional_t<KV8, uint8_t, float>;
     auto load_scale = [&](int it, const float* sc) {
         if constexpr (KV8) {
-            if (tid < C::KEYS) rsc = sc[slot_of(min(it * C::KEYS + tid, maxpos)) * p.nkv + kh];
+            if (tid < C::KEYS) {
+                const int t0 = min(it * KS + (tid >> 5), maxpos >> 5);
+                rsc = sc[((size_t)tslot[t0] + min(tid & 31, maxpos - 32 * t0)) * p.nkv + kh];
+            }
         }
     };
+    // K: thread t takes chunk t % CPK of keys t / CPK + u * KPT. A wave's keys
+    // of one u lie in one tile.
+    constexpr int KPT = C::NT / CPK;
+    static_assert(64 / CPK <= 32 && KPT * CPK == C::NT, "a wave's keys lie in one tile");
+    const int kkey = tid / CPK;
+    const uint32_t kcol = 8 * (tid % CPK);
     auto load_k = [&](int it) {
 #pragma unroll
         for (int u = 0; u < C::NKC; ++u) {
-            int key, c;
-            const size_t o = kaddr(it, u, key, c);
+            const TileAt t = tile_at(it, __builtin_amdgcn_readfirstlane((kkey + u * KPT) >> 5));
+            const Elem* src = static_cast<const Elem*>(p.kc) + t.base;
+            const uint32_t o = __umul24((uint32_t)min((kkey + u * KPT) & 31, t.last), (uint32_t)p.hkv) + kcol;
             if constexpr (KV8) {
-                const uint2 v = *reinterpret_cast<const uint2*>(static_cast<const uint8_t*>(p.kc) + o);
+                const uint2 v = *reinterpret_cast<const uint2*>(src + o);
                 r8[2 * u] = v.x;
                 r8[2 * u + 1] = v.y;
             } else {
-                const float4* src = reinterpret_cast<const float4*>(static_cast<const float*>(p.kc) + o);
-                rf[2 * u] = src[0];
-                rf[2 * u + 1] = src[1];
+                rf[2 * u] = *reinterpret_cast<const float4*>(src + o);
+                rf[2 * u + 1] = *reinterpret_cast<const float4*>(src + o + 4);
             }
         }
         load_scale(it, p.ks);
-    };
-    // LDS: K part t of tile w: [32 keys][HD] bf16, 16-byte chunk c of key r at
-    // c ^ (r & 15) (HD 64: c ^ (r >> 1 & 7)), so the 16 lanes of a fragment
-    // read on 16 rows hit 16 slots of a bank line.
-    auto kchunk = [&](int r, int c) -> int {
-        return r * (HD * 2) + ((HD == 128 ? c ^ (r & 15) : c ^ ((r >> 1) & 7)) << 4);
     };
     auto store_k = [&]() {
 #pragma unroll
@@ -200,20 +245,27 @@ __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p)
     // A V block: 8 keys of one k-half of a 16-key step (the keys that half of
     // the lanes holds of the scores: 4h..4h+3 and 8+4h..8+4h+3) x 4 d.
     constexpr int DG = HD / 4;
-    auto vkey = [&](int oct, int j) -> int {  // octet of the step -> key of the step
-        const int in = oct & 3;
-        return 32 * (oct >> 2) + 16 * (in >> 1) + 4 * (in & 1) + (j < 4 ? j : 4 + j);
-    };
+    static_assert(4 * DG >= 64, "a wave's octets lie in one tile");
     auto load_v = [&](int it) {
 #pragma unroll
         for (int u = 0; u < C::NVB; ++u) {
             const int q = tid + u * C::NT, oct = q / DG, dg = q % DG;
             if (C::VB < C::NT && tid >= C::VB) break;
+            const TileAt t = tile_at(it, __builtin_amdgcn_readfirstlane(oct >> 2));
+            const Elem* src = static_cast<const Elem*>(p.vc) + t.base;
+            const int k0 = 16 * ((oct >> 1) & 1) + 4 * (oct & 1);
+            auto at = [&](int j, const Elem* v) {
+                if constexpr (KV8) r8[8 * u + j] = *reinterpret_cast<const uint32_t*>(v);
+                else rf[8 * u + j] = *reinterpret_cast<const float4*>(v);
+            };
+            if (t.last == 31) {  // a uniform row stride: one lane offset for the eight loads
+                const uint32_t o = __umul24((uint32_t)k0, (uint32_t)p.hkv) + 4 * dg;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const size_t o = slot_of(min(it * C::KEYS + vkey(oct, j), maxpos)) * p.hkv + (size_t)kh * HD + 4 * dg;
-                if constexpr (KV8) r8[8 * u + j] = *reinterpret_cast<const uint32_t*>(static_cast<const uint8_t*>(p.vc) + o);
-                else rf[8 * u + j] = *reinterpret_cast<const float4*>(static_cast<const float*>(p.vc) + o);
+                for (int j = 0; j < 8; ++j) at(j, src + (size_t)((j < 4 ? j : 4 + j) * p.hkv) + o);
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    at(j, src + (__umul24((uint32_t)min(k0 + (j < 4 ? j : 4 + j), t.last), (uint32_t)p.hkv) + 4 * dg));
             }
         }
         load_scale(it, p.vs);
@@ -268,7 +320,8 @@ __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p)
     for (int j = 0; j < HD / 32; ++j)
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[j][e] = 0.0f;
-    float m = -INFINITY, l = 0.0f;  // l: this half's keys only
+    const float c2 = p.scale * 1.44269504088896341f;
+    float m = NO_REF, l = 0.0f;  // l: this half's keys only
 
     load_k(0);
     for (int it = 0; it < niter; ++it) {
@@ -283,24 +336,31 @@ __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p)
 #pragma unroll
             for (int e = 0; e < 16; ++e) s[e] = 0.0f;
             const uint8_t* kb = lds + ks * C::PARTS * C::TILE;
+            // The small partial products first: only the HD / 16 sums of
+            // k1q1 then round at the size of the score.
 #pragma unroll
             for (int t = 0; t < HD / 16; ++t) {
                 const uint8_t* src = kb + kchunk(col, 2 * t + half);
                 const v4i k1 = *reinterpret_cast<const v4i*>(src);
+                const v4i qt = *reinterpret_cast<const v4i*>(q3w + kchunk(col, 2 * t + half));
                 if constexpr (KV8) {
-                    s = mfma(k1, qf[t][2], s);
+                    s = mfma(k1, qt, s);
                     s = mfma(k1, qf[t][1], s);
                     s = mfma(k1, qf[t][0], s);
                 } else {
                     const v4i k2 = *reinterpret_cast<const v4i*>(src + C::TILE);
                     const v4i k3 = *reinterpret_cast<const v4i*>(src + 2 * C::TILE);
                     s = mfma(k3, qf[t][0], s);
-                    s = mfma(k1, qf[t][2], s);
+                    s = mfma(k1, qt, s);
                     s = mfma(k2, qf[t][1], s);
                     s = mfma(k2, qf[t][0], s);
                     s = mfma(k1, qf[t][1], s);
-                    s = mfma(k1, qf[t][0], s);
                 }
+            }
+            if constexpr (!KV8) {
+#pragma unroll
+                for (int t = 0; t < HD / 16; ++t)
+                    s = mfma(*reinterpret_cast<const v4i*>(kb + kchunk(col, 2 * t + half)), qf[t][0], s);
             }
             // Register e: key 8 (e / 4) + 4 half + e % 4 of the tile.
             if constexpr (KV8) {
@@ -313,22 +373,20 @@ __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p)
                     s[4 * e4 + 3] = s[4 * e4 + 3] * k.w;
                 }
             }
-#pragma unroll
-            for (int e = 0; e < 16; ++e) s[e] = s[e] * p.scale;
             if (j0 + 31 > wminpos) {
                 const int lim = mypos - j0 - 4 * half;  // keys of this half up to here are visible
 #pragma unroll
                 for (int e = 0; e < 16; ++e)
-                    if (8 * (e >> 2) + (e & 3) > lim) s[e] = -INFINITY;
+                    if (8 * (e >> 2) + (e & 3) > lim) s[e] = MASKED;
             }
             float mx = s[0];
 #pragma unroll
             for (int e = 1; e < 16; ++e) mx = fmaxf(mx, s[e]);
-            mx = fmaxf(mx, xor_lane<32>(mx));
-            const float mn = fmaxf(m, mx);
-            const float ref = mn == -INFINITY ? 0.0f : mn;  // no key seen yet: every weight is 0
-            if (__any(mn != m)) {
-                const float alpha = expf(m - ref);
+            mx = fmaxf(mx, xor_lane<32>(mx)) * c2;  // c2 > 0: the largest scaled score
+            const bool up = mx > m + SLACK;
+            if (__any(up)) {
+                const float mn = up ? mx : m;
+                const float alpha = __builtin_amdgcn_exp2f(m - mn);  // 1 where the reference stays
                 l = l * alpha;
 #pragma unroll
                 for (int j = 0; j < HD / 32; ++j)
@@ -339,7 +397,7 @@ __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p)
             float sum = 0.0f;
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
-                s[e] = expf(s[e] - ref);
+                s[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[e], c2, -m));
                 sum = sum + s[e];
             }
             l = l + sum;
@@ -360,32 +418,48 @@ __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p)
                 }
             }
             const uint8_t* vb = lds + C::VOFF + ks * C::PARTS * C::TILE;
+            v4i pf[2][3];
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
                 float x[8];
 #pragma unroll
                 for (int i = 0; i < 8; ++i) x[i] = s[8 * t + i];
-                v4i p1, p2, p3;
-                split8(x, p1, p2, p3);
+                split8(x, pf[t][0], pf[t][1], pf[t][2]);
+            }
 #pragma unroll
-                for (int j = 0; j < HD / 32; ++j) {
-                    const int d = 32 * j + col;
-                    const uint8_t* src = vb + vchunk(d >> 2, d & 3, 2 * t + half);
-                    const v4i v1 = *reinterpret_cast<const v4i*>(src);
-                    if constexpr (KV8) {
-                        o[j] = mfma(v1, p3, o[j]);
-                        o[j] = mfma(v1, p2, o[j]);
-                        o[j] = mfma(v1, p1, o[j]);
-                    } else {
-                        const v4i v2 = *reinterpret_cast<const v4i*>(src + C::TILE);
-                        const v4i v3 = *reinterpret_cast<const v4i*>(src + 2 * C::TILE);
-                        o[j] = mfma(v3, p1, o[j]);
-                        o[j] = mfma(v1, p3, o[j]);
-                        o[j] = mfma(v2, p2, o[j]);
-                        o[j] = mfma(v2, p1, o[j]);
-                        o[j] = mfma(v1, p2, o[j]);
-                        o[j] = mfma(v1, p1, o[j]);
+            for (int j = 0; j < HD / 32; ++j) {
+                const int d = 32 * j + col;
+                const uint8_t* src[2] = {vb + vchunk(d >> 2, d & 3, half), vb + vchunk(d >> 2, d & 3, 2 + half)};
+                if constexpr (KV8) {
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) {
+                        const v4i v1 = *reinterpret_cast<const v4i*>(src[t]);
+                        o[j] = mfma(v1, pf[t][2], o[j]);
+                        o[j] = mfma(v1, pf[t][1], o[j]);
+                        o[j] = mfma(v1, pf[t][0], o[j]);
                     }
+                } else {
+                    // The tile's sum on its own, small products first, then
+                    // one addition to the context.
+                    v16f a;
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) a[e] = 0.0f;
+                    v4i v1[2];
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) {
+                        v1[t] = *reinterpret_cast<const v4i*>(src[t]);
+                        const v4i v2 = *reinterpret_cast<const v4i*>(src[t] + C::TILE);
+                        const v4i v3 = *reinterpret_cast<const v4i*>(src[t] + 2 * C::TILE);
+                        a = mfma(v3, pf[t][0], a);
+                        a = mfma(v1[t], pf[t][2], a);
+                        a = mfma(v2, pf[t][1], a);
+                        a = mfma(v2, pf[t][0], a);
+                        a = mfma(v1[t], pf[t][1], a);
+                    }
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) a = mfma(v1[t], pf[t][0], a);
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) o[j][e] = o[j][e] + a[e];
                 }
             }
         }
@@ -409,8 +483,8 @@ __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p)
         barrier();
         if (ks < w) {
             const float m2 = sml[(ks % w) * QG + qg][0][lane], l2 = sml[(ks % w) * QG + qg][1][lane];
-            const float mn = fmaxf(m, m2), ref = mn == -INFINITY ? 0.0f : mn;
-            const float a1 = expf(m - ref), a2 = expf(m2 - ref);
+            const float mn = fmaxf(m, m2);
+            const float a1 = __builtin_amdgcn_exp2f(m - mn), a2 = __builtin_amdgcn_exp2f(m2 - mn);
             m = mn;
             l = l * a1 + l2 * a2;
 #pragma unroll
@@ -451,8 +525,8 @@ hipError_t go(hipStream_t s, const FlashArgs& a) {
 
 hipError_t launch_flash_prefill(hipStream_t s, const FlashArgs& a, int hd, bool kv8) {
     if (a.rows_per_seq <= 0 || a.nseq <= 0) return hipSuccess;
-    if (hd == 128) return kv8 ? go<true, 128, 2, 4>(s, a) : go<false, 128, 2, 4>(s, a);
-    return kv8 ? go<true, 64, 2, 4>(s, a) : go<false, 64, 2, 4>(s, a);
+    if (hd == 128) return kv8 ? go<true, 128, 2, 4>(s, a) : go<false, 128, 2, 2>(s, a);
+    return kv8 ? go<true, 64, 2, 4>(s, a) : go<false, 64, 2, 2>(s, a);
 }
 
 }  // namespace bh

@@ -1536,7 +1536,7 @@ int bh_qwen3_create(const bh_qwen3_config* cfg, uint32_t max_batch, uint32_t max
     e->tmpw_floats = std::max<uint64_t>(std::max<uint64_t>((uint64_t)e->W * d, 2 * ff * d), d * std::max<uint64_t>(hq, ff));
     if (!c.tie_embeddings) e->tmpw_floats = std::max<uint64_t>(e->tmpw_floats, (uint64_t)c.vocab * d);
     const uint64_t R = max_rows;
-    e->flash = flash_ok((int)c.head_dim, (int)c.n_heads, (int)c.n_kv_heads, (int)e->kv_max_bt);
+    e->flash = flash_ok((int)c.head_dim, (int)c.n_heads, (int)c.n_kv_heads, (int)max_seq);
     const uint64_t PR = e->flash ? max_batch : R;  // rows of chunk partials: decode rows, or prompt rows too
     if ((rc = dalloc(e, &e->emb, (uint64_t)c.vocab * d)) || (rc = dalloc(e, &e->norm, d)) ||
         (rc = dalloc(e, &e->head, (uint64_t)c.vocab * d / 4)) || (rc = dalloc(e, &e->shead, c.vocab)) ||

@@ -1,0 +1,121 @@
+"""The prompt attention kernel (bh::launch_flash_prefill, which the Qwen3 engine
+runs for every prefill chunk) against 64-bit softmax attention: row counts
+around the 32-vector wave and the workgroup, positions around the 32-key tile
+and the KS-tile step, every group size, both head widths, both caches, slabs
+and a shuffled paged pool; and its independence of how a prompt is chunked.
+
+Tolerance: a score is a dot product of head_dim f32 products, so its error is
+up to head_dim * 2^-24 of sum |q||k| scale; that error is the relative error
+of a weight. With normal q and k (|q||k| summed over head_dim * scale is about
+0.64 * sqrt(head_dim)) this is 128 * 6e-8 * 7 = 5e-5 at worst and about
+sqrt(head_dim) * 6e-8 * 7 = 5e-6 as rounding errors add up; the bar is 1e-5 in
+the 2-norm, and the largest error that f32 arithmetic of the plain formula
+shows on the same data times 2."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+from brain_amd import load
+
+pytestmark = pytest.mark.gpu
+
+
+class KvMap(C.Structure):
+    _fields_ = [("bt", C.c_void_p), ("max_bt", C.c_int), ("bs", C.c_int), ("nblk", C.c_int), ("max_seq", C.c_int)]
+
+
+class FlashArgs(C.Structure):
+    _fields_ = [(n, C.c_void_p) for n in ("q", "kc", "vc", "ks", "vs", "pos", "seq")] + \
+               [(n, C.c_int) for n in ("nh", "nkv", "hq", "hkv", "rows_per_seq", "nseq")] + \
+               [("scale", C.c_float), ("map", KvMap)]
+
+
+def flash():
+    fn = getattr(load(), "_ZN2bh20launch_flash_prefillEP12ihipStream_tRKNS_9FlashArgsEib")
+    fn.restype, fn.argtypes = C.c_int, [C.c_void_p, C.POINTER(FlashArgs), C.c_int, C.c_bool]
+    return fn
+
+
+class Setup:
+    def __init__(self, nseq, npos, nkv, group, hd, kv8, paged, seed=0):
+        g = torch.Generator(device="cuda")
+        g.manual_seed(seed)
+        self.nseq, self.nkv, self.group, self.hd, self.kv8 = nseq, nkv, group, hd, kv8
+        self.nh, self.max_seq = nkv * group, npos + 3
+        hkv = nkv * hd
+        if paged:
+            bs = 32 if npos < 300 else 96
+            self.max_bt = (self.max_seq + bs - 1) // bs
+            self.nblk = nseq * self.max_bt + 1
+            bt = torch.randperm(self.nblk, device="cuda", generator=g)[: nseq * self.max_bt].view(nseq, -1)
+            slots, self.bs = self.nblk * bs, bs
+            self.bt = bt.to(torch.int32).contiguous()
+            at = torch.arange(npos, device="cuda")
+            self.slot = bt[:, at // bs] * bs + at % bs
+        else:
+            self.bt, self.bs, self.max_bt, self.nblk = None, 0, 0, 0
+            slots = nseq * self.max_seq
+            self.slot = torch.arange(nseq, device="cuda")[:, None] * self.max_seq + torch.arange(npos, device="cuda")
+        if kv8:
+            self.k, self.v = (torch.randint(-127, 128, (slots, hkv), device="cuda", generator=g, dtype=torch.int8) for _ in "kv")
+            self.ks, self.vs = ((torch.rand(slots, nkv, device="cuda", generator=g) + 0.5) / 70 for _ in "kv")
+        else:
+            self.k, self.v = (torch.randn(slots, hkv, device="cuda", generator=g) for _ in "kv")
+            self.ks = self.vs = None
+        self.q = torch.randn(nseq, npos, self.nh, hd, device="cuda", generator=g)
+
+    def run(self, p0, p1):
+        """Context of rows p0..p1 of every sequence."""
+        n = p1 - p0
+        q = self.q[:, p0:p1].clone(memory_format=torch.contiguous_format)  # the kernel writes over it
+        pos = torch.arange(p0, p1, device="cuda", dtype=torch.int32).repeat(self.nseq)
+        seq = torch.arange(self.nseq, device="cuda", dtype=torch.int32).repeat_interleave(n)
+        ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
+        a = FlashArgs(q.data_ptr(), ptr(self.k), ptr(self.v), ptr(self.ks), ptr(self.vs), pos.data_ptr(), seq.data_ptr(),
+                      self.nh, self.nkv, self.nh * self.hd, self.nkv * self.hd, n, self.nseq, self.hd ** -0.5,
+                      KvMap(ptr(self.bt), self.max_bt, self.bs, self.nblk, self.max_seq))
+        rc = flash()(torch.cuda.current_stream().cuda_stream, C.byref(a), self.hd, self.kv8)
+        assert rc == 0
+        torch.cuda.synchronize()
+        return q
+
+    def ref(self, p0, p1, dtype):
+        out = torch.empty(self.nseq, p1 - p0, self.nh, self.hd, device="cuda", dtype=dtype)
+        mask = torch.arange(p1, device="cuda")[None, :] > torch.arange(p0, p1, device="cuda")[:, None]
+        for b in range(self.nseq):
+            sl = self.slot[b, :p1]
+            k, v = (x[sl].to(dtype).view(p1, self.nkv, self.hd) for x in (self.k, self.v))
+            if self.kv8:
+                k, v = k * self.ks[sl].to(dtype)[:, :, None], v * self.vs[sl].to(dtype)[:, :, None]
+            for h in range(self.nh):
+                s = (self.q[b, p0:p1, h].to(dtype) @ k[:, h // self.group].t()) * self.hd ** -0.5
+                out[b, :, h] = torch.softmax(s.masked_fill(mask, -float("inf")), -1) @ v[:, h // self.group]
+        return out
+
+
+@pytest.mark.parametrize("kv8", [False, True])
+@pytest.mark.parametrize("nseq,npos,nkv,group,hd,paged", [
+    (1, 1, 1, 1, 128, False), (2, 15, 2, 2, 64, False), (1, 33, 2, 4, 128, True), (3, 64, 1, 8, 64, True),
+    (1, 127, 1, 3, 128, False), (2, 129, 2, 5, 64, True), (1, 257, 1, 7, 128, True), (1, 1030, 2, 2, 128, False),
+    (2, 515, 1, 6, 64, False),
+])
+def test_flash_prefill_matches_softmax(gpu, kv8, nseq, npos, nkv, group, hd, paged):
+    s = Setup(nseq, npos, nkv, group, hd, kv8, paged, seed=npos)
+    for p0, p1 in {(0, npos), (npos // 3, npos), (npos - 1, npos)}:
+        got, want = s.run(p0, p1).double(), s.ref(p0, p1, torch.float64)
+        err = (got - want).norm() / want.norm()
+        assert err < 1e-5, (p0, p1, float(err))
+        plain = (s.ref(p0, p1, torch.float32).double() - want).abs().max()
+        assert (got - want).abs().max() < 2 * plain + 1e-6, (p0, p1, float((got - want).abs().max()), float(plain))
+
+
+@pytest.mark.parametrize("kv8", [False, True])
+@pytest.mark.parametrize("hd,group", [(128, 2), (64, 5)])
+def test_flash_prefill_chunking_gives_the_same_bits(gpu, kv8, hd, group):
+    s = Setup(2, 300, 2, group, hd, kv8, True, seed=9)
+    whole = s.run(0, 300)
+    cuts = [0, 1, 2, 35, 64, 191, 300]
+    parts = torch.cat([s.run(a, b) for a, b in zip(cuts, cuts[1:])], 1)
+    assert torch.equal(whole, parts)
