@@ -48,7 +48,7 @@ hipError_t launch_gemm_i8_noalloc(hipStream_t s, const uint32_t* xq, const uint3
                                   const float* sw, const float* bias, void* out, int out_dtype, int m, int kg, int n,
                                   size_t* need_bytes);
 size_t noalloc_scratch_bytes();
-size_t gemm_q4_workspace_ints(int m, int k, int n);
+size_t gemm_pad_workspace_ints(int m, int kg, int n);
 hipError_t launch_gemv_i8_gated(hipStream_t s, const uint32_t* xq, const uint32_t* wq, const float* sx,
                                 const float* sw, const float* gate, int gate_stride, int gate_col, float* out, int m,
                                 int kg, int n);
@@ -367,12 +367,13 @@ int bh_matmul_i8_dyn_noalloc(void* stream, const uint32_t* xq, const uint32_t* w
 int bh_reserve_workspace(void* stream, uint32_t m, uint32_t kg, uint32_t n) {
     if ((uint64_t)kg * 4 > I32MAX || m > I32MAX || n > I32MAX)
         return fail(BH_ERR_INVALID, "bh_reserve_workspace: m=%u kg=%u n=%u out of range", m, kg, n);
-    // Both workspaces a GEMM of this shape may take: the split-K slabs of the
-    // int8 GEMM (bh_matmul_i8_dyn or bh_matmul_i8_dyn_quant), and for W4A8
-    // (K = 4*kg) the weights expanded to int8.
-    const size_t need[2] = {std::max(gemm_workspace_ints((int)m, (int)kg, (int)n),
-                                     gemm_quant_workspace_ints((int)m, (int)kg, (int)n)),
-                            gemm_q4_workspace_ints((int)m, (int)kg * 4, (int)n)};
+    // Both workspaces a GEMM of this shape may take: the split-K slabs
+    // (bh_matmul_i8_dyn, bh_matmul_i8_dyn_quant, W4A8) and, for K % 128 != 0,
+    // the zero-padded operands (whose GEMM is the padded shape's).
+    const size_t pad = gemm_pad_workspace_ints((int)m, (int)kg, (int)n);
+    size_t split = std::max(gemm_workspace_ints((int)m, (int)kg, (int)n), gemm_quant_workspace_ints((int)m, (int)kg, (int)n));
+    if (pad) split = std::max(split, gemm_workspace_ints((int)m, ((int)kg + 31) / 32 * 32, (int)n));
+    const size_t need[2] = {split, pad};
     for (int slot = 0; slot < 2; ++slot) {
         if (!need[slot]) continue;
         hipError_t err = hipSuccess;

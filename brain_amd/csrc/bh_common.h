@@ -127,6 +127,16 @@ __device__ __forceinline__ void unpack_q4x4(v4i w, v4i& a, v4i& b) {
     b = v4i{(int)l2, (int)h2, (int)l3, (int)h3};
 }
 
+// 8 bytes of int4 (16 K values) -> 16 int8 holding 16 q each: a nibble moved to
+// the top of its byte is 16 times its two's complement value, so no sign
+// extension is needed. The sums come out 16 times too large, exactly.
+__device__ __forceinline__ v4i unpack_q4_x16(uint2 w) {
+    const uint32_t e0 = (w.x << 4) & 0xF0F0F0F0u, o0 = w.x & 0xF0F0F0F0u;  // nibbles 0,2,4,6 and 1,3,5,7
+    const uint32_t e1 = (w.y << 4) & 0xF0F0F0F0u, o1 = w.y & 0xF0F0F0F0u;
+    return v4i{(int)__builtin_amdgcn_perm(o0, e0, 0x05010400u), (int)__builtin_amdgcn_perm(o0, e0, 0x07030602u),
+               (int)__builtin_amdgcn_perm(o1, e1, 0x05010400u), (int)__builtin_amdgcn_perm(o1, e1, 0x07030602u)};
+}
+
 // The dequant epilogue of matmul_i8_dyn / matmul_i8_gemv: (f32(acc)*sx)*sw,
 // evaluated left to right with no fused multiply-add (the library is built
 // with -ffp-contract=off), then the optional bias add.

@@ -26,6 +26,7 @@
 #include <cstdlib>
 
 #include <mutex>
+#include <type_traits>
 
 #include "bh_common.h"
 
@@ -331,7 +332,8 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_i8_kernel(GemmArgs a) {
 // the epilogue writes with one 8-byte (bf16) or 16-byte (f32) store.
 template <int DK>
 __device__ __forceinline__ int dswz(int r) {
-    if constexpr (DK == 64) return (r >> 2) & 3;
+    if constexpr (DK == 32) return (r >> 3) & 1;
+    else if constexpr (DK == 64) return (r >> 2) & 3;
     else if constexpr (DK == 128) return (r >> 1) & 7;
     else return r & 15;  // DK = 256: a row is one whole 256-byte bank line
 }
@@ -345,13 +347,17 @@ __device__ __forceinline__ void wait_vmcnt() {
     __builtin_amdgcn_s_waitcnt((N & 0xF) | (0x7 << 4) | (0xF << 8) | ((N >> 4) << 14));
 }
 
-template <int BM, int BN, int WM, int WN, int STAGES, int DK>
+// Q4: the weight operand is int4 (W4A8, [N, K/8] u32): its LDS rows are DK / 2
+// bytes and a fragment is 8 bytes of it, unpacked on the way to the MFMA.
+template <int BM, int BN, int WM, int WN, int STAGES, int DK, bool Q4 = false>
 struct DmaCfg {
+    static constexpr int BDK = Q4 ? DK / 2 : DK;  // bytes of a B row per stage
+    static constexpr int BCPR = BDK / 16;
     static constexpr int NT = WM * WN * 64;
     static constexpr int WTM = BM / WM, WTN = BN / WN;
     static constexpr int FM = WTM / 32, FN = WTN / 32;
     static constexpr int CPR = DK / 16;  // 16-byte chunks per LDS row
-    static constexpr int A_BYTES = BM * DK, B_BYTES = BN * DK;
+    static constexpr int A_BYTES = BM * DK, B_BYTES = BN * BDK;
     static constexpr int STAGE = A_BYTES + B_BYTES;
     static constexpr int A_LOADS = A_BYTES / 16 / NT;  // DMA instructions per thread per stage
     static constexpr int B_LOADS = B_BYTES / 16 / NT;
@@ -379,10 +385,10 @@ __device__ __forceinline__ void wait_ahead(int ahead) {
 }
 
 template <int BM, int BN, int WM, int WN, int STAGES, int DK, int OUT, bool HAS_BIAS, bool STATIC, bool SPLITK,
-          bool ILV_ENABLE = false, bool PP = false>
+          bool ILV_ENABLE = false, bool PP = false, bool Q4 = false>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_i8_dma_kernel(GemmArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the LDS-DMA builtins exist only in the device pass
-    using C = DmaCfg<BM, BN, WM, WN, STAGES, DK>;
+    using C = DmaCfg<BM, BN, WM, WN, STAGES, DK, Q4>;
     __shared__ __attribute__((aligned(1024))) uint8_t lds[STAGES * C::STAGE];
 
     const int m = a.m, n = a.n;
@@ -422,9 +428,10 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_i8_dma_kernel(GemmArgs a) {
     }
 #pragma unroll
     for (int i = 0; i < C::B_LOADS; ++i) {
-        const int q = t + C::NT * i, r = q / C::CPR, p = q % C::CPR;
+        const int q = t + C::NT * i, r = q / C::BCPR, p = q % C::BCPR;
         const int gr = min(col0 + r, n - 1);
-        bsrc[i] = reinterpret_cast<const uint8_t*>(a.wq) + (int64_t)gr * kbytes + ((p ^ dswz<DK>(r)) << 4);
+        bsrc[i] = reinterpret_cast<const uint8_t*>(a.wq) + (int64_t)gr * (Q4 ? kbytes / 2 : kbytes) +
+                  ((p ^ dswz<C::BDK>(r)) << 4);
     }
     // The wave-uniform LDS base of load i (the hardware adds lane*16). The
     // DMA is issued through inline asm so the compiler does not track it:
@@ -439,11 +446,11 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_i8_dma_kernel(GemmArgs a) {
     };
     auto issue = [&](int kt, int buf) {
         const uint32_t base = lds_base + buf * C::STAGE;
-        const int64_t koff = (int64_t)kt * DK;
+        const int64_t koff = (int64_t)kt * DK, bkoff = (int64_t)kt * C::BDK;
 #pragma unroll
         for (int i = 0; i < C::A_LOADS; ++i) dma(asrc[i] + koff, base + i * C::NT * 16);
 #pragma unroll
-        for (int i = 0; i < C::B_LOADS; ++i) dma(bsrc[i] + koff, base + C::A_BYTES + i * C::NT * 16);
+        for (int i = 0; i < C::B_LOADS; ++i) dma(bsrc[i] + bkoff, base + C::A_BYTES + i * C::NT * 16);
     };
 
     // Epilogue operands of this tile (column scales and bias, row scales and
@@ -488,23 +495,51 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_i8_dma_kernel(GemmArgs a) {
         if (s < nk) issue(kt0 + s, s);
 
     const int frow = lane & 31, fchk = lane >> 5;
-    auto read_frags = [&](const uint8_t* A, int ks, v4i* fa, v4i* fb) {
+    // A B fragment as it waits for its MFMAs. Q4 with several MFMAs a step: the
+    // 8 bytes read, unpacked between the MFMAs of the step (512x4096x11008 on
+    // 256x128 tiles 40.9 -> 39.0 us); with one MFMA a step there is no between,
+    // and it is unpacked as it is read (128x4096x11008 on 64x64 tiles 30.9 us
+    // against 33.6).
+    constexpr bool LAZY = Q4 && C::FM > 1;
+    using FragB = std::conditional_t<LAZY, uint2, v4i>;
+    auto whole = [](const FragB& f) -> v4i {
+        if constexpr (LAZY) return unpack_q4_x16(f);
+        else return f;
+    };
+    auto read_frags = [&](const uint8_t* A, int ks, v4i* fa, FragB* fb) {
         const uint8_t* B = A + C::A_BYTES;
 #pragma unroll
         for (int i = 0; i < C::FM; ++i)
             fa[i] = *reinterpret_cast<const v4i*>(A + dslot<DK>(wm * C::WTM + i * 32 + frow, 2 * ks + fchk));
 #pragma unroll
-        for (int j = 0; j < C::FN; ++j)
-            fb[j] = *reinterpret_cast<const v4i*>(B + dslot<DK>(wn * C::WTN + j * 32 + frow, 2 * ks + fchk));
+        for (int j = 0; j < C::FN; ++j) {
+            const int r = wn * C::WTN + j * 32 + frow;
+            if constexpr (Q4) {
+                const uint2 w = *reinterpret_cast<const uint2*>(B + dslot<C::BDK>(r, ks) + 8 * fchk);
+                if constexpr (LAZY) fb[j] = w;
+                else fb[j] = unpack_q4_x16(w);
+            }
+            else fb[j] = *reinterpret_cast<const v4i*>(B + dslot<DK>(r, 2 * ks + fchk));
+        }
     };
     // One k-step of MFMAs with the next k-step's fragment reads interleaved:
     // MFMA, read, MFMA, read, ... then the remaining MFMAs.
-    auto mfma_step = [&](const v4i* fa, const v4i* fb) {
+    auto mfma_step = [&](const v4i* fa, const FragB* fb) {
+        if constexpr (LAZY) {
 #pragma unroll
-        for (int i = 0; i < C::FM; ++i)
+            for (int j = 0; j < C::FN; ++j) {
+                const v4i b = whole(fb[j]);
 #pragma unroll
-            for (int j = 0; j < C::FN; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb[j], fa[i], acc[i][j], 0, 0, 0);
+                for (int i = 0; i < C::FM; ++i)
+                    acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(b, fa[i], acc[i][j], 0, 0, 0);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < C::FM; ++i)
+#pragma unroll
+                for (int j = 0; j < C::FN; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb[j], fa[i], acc[i][j], 0, 0, 0);
+        }
     };
     auto interleave = [&]() {
 #pragma unroll
@@ -526,12 +561,12 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_i8_dma_kernel(GemmArgs a) {
         if (idx < C::A_LOADS) dma(asrc[idx] + koff, base + idx * C::NT * 16);
         else dma(bsrc[idx - C::A_LOADS] + koff, base + C::A_BYTES + (idx - C::A_LOADS) * C::NT * 16);
     };
-    auto mfma_range = [&](const v4i* fa_, const v4i* fb_, int q0, int cnt) {
+    auto mfma_range = [&](const v4i* fa_, const FragB* fb_, int q0, int cnt) {
 #pragma unroll
         for (int q = 0; q < C::FM * C::FN; ++q) {
             if (q < q0 || q >= q0 + cnt) continue;
             const int i = q / C::FN, j = q % C::FN;
-            acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb_[j], fa_[i], acc[i][j], 0, 0, 0);
+            acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(whole(fb_[j]), fa_[i], acc[i][j], 0, 0, 0);
         }
     };
     auto interleave_reads = [&]() {
@@ -562,6 +597,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_i8_dma_kernel(GemmArgs a) {
         // branches: a barrier under an exec mask would still execute.
         const int grp = __builtin_amdgcn_readfirstlane(wave) >> 2;
         v4i pa[C::KSTEPS][C::FM], pb[C::KSTEPS][C::FN];
+        FragB praw[C::KSTEPS][C::FN];
         // Stage 0 complete (every wave's share) before group 0's first L.
         if (nk > 0) wait_ahead<C::LOADS, STAGES - 2>(min(nk - 1, STAGES - 2));
         __builtin_amdgcn_sched_barrier(0);
@@ -576,9 +612,13 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_i8_dma_kernel(GemmArgs a) {
             else wait_ahead<C::LOADS, STAGES - 3>(min(nk - 2 - it, STAGES - 3));
             const uint8_t* A = lds + (it % STAGES) * C::STAGE;
 #pragma unroll
-            for (int ks = 0; ks < C::KSTEPS; ++ks) read_frags(A, ks, pa[ks], pb[ks]);
+            for (int ks = 0; ks < C::KSTEPS; ++ks) read_frags(A, ks, pa[ks], praw[ks]);
             if (it + STAGES - 1 < nk) issue(kt0 + it + STAGES - 1, (it + STAGES - 1) % STAGES);
             __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the fragments are in registers
+#pragma unroll
+            for (int ks = 0; ks < C::KSTEPS; ++ks)
+#pragma unroll
+                for (int j = 0; j < C::FN; ++j) pb[ks][j] = whole(praw[ks][j]);
             __builtin_amdgcn_sched_barrier(0);
             __builtin_amdgcn_s_barrier();
             __builtin_amdgcn_sched_barrier(0);
@@ -599,7 +639,8 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_i8_dma_kernel(GemmArgs a) {
             __builtin_amdgcn_sched_barrier(0);
         }
     } else {
-    v4i fa[2][C::FM], fb[2][C::FN];
+    v4i fa[2][C::FM];
+    FragB fb[2][C::FN];
     if (nk > 0) {
         wait_ahead<C::LOADS, STAGES - 2>(min(nk - 1, STAGES - 2));
         __builtin_amdgcn_s_barrier();
@@ -641,7 +682,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_i8_dma_kernel(GemmArgs a) {
                 }
             } else {
                 mfma_step(fa[cur], fb[cur]);
-                interleave();
+                if constexpr (!LAZY) interleave();
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -656,6 +697,14 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_i8_dma_kernel(GemmArgs a) {
 
     }
 
+    if constexpr (Q4) {  // the weights went in as 16 q: exact, as is the division
+#pragma unroll
+        for (int i = 0; i < C::FM; ++i)
+#pragma unroll
+            for (int j = 0; j < C::FN; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[i][j][e] >>= 4;
+    }
     // Lane l, register e of fragment (i,j): row rbase + 32i, columns
     // cbase + 32j + 8*(e/4) + (e%4).
     const int rbase = row0 + wm * C::WTM + (lane & 31);
@@ -955,6 +1004,9 @@ static int t32x64_env() {
     return v;
 }
 
+// Sums of int8 x 16 q stay inside i32 below this K: K * 128 * 8 * 16 < 2^31.
+constexpr int Q4_MAX_K = 131072;
+
 constexpr size_t SPLITK_MAX_BYTES = size_t(64) << 20;  // workspace cap per call
 
 // Split-K. Measured on MI355X, a tile alone on its CU costs a few us fixed
@@ -1064,11 +1116,11 @@ static hipError_t go(hipStream_t s, bool aligned, const GemmArgs& a) {
 }
 
 template <int BM, int BN, int WM, int WN, int STAGES, int DK, int OUT, bool HAS_BIAS, bool STATIC, bool SPLITK,
-          bool ILV = false, bool PP = false>
+          bool ILV = false, bool PP = false, bool Q4 = false>
 static hipError_t go_dma(hipStream_t s, const GemmArgs& a) {
     const long tiles = (long)((a.m + BM - 1) / BM) * ((a.n + BN - 1) / BN);
     const unsigned grid = (unsigned)(tiles * (SPLITK ? a.splits : 1));
-    gemm_i8_dma_kernel<BM, BN, WM, WN, STAGES, DK, OUT, HAS_BIAS, STATIC, SPLITK, ILV, PP><<<grid, WM * WN * 64, 0, s>>>(a);
+    gemm_i8_dma_kernel<BM, BN, WM, WN, STAGES, DK, OUT, HAS_BIAS, STATIC, SPLITK, ILV, PP, Q4><<<grid, WM * WN * 64, 0, s>>>(a);
     return hipGetLastError();
 }
 
@@ -1173,6 +1225,27 @@ hipError_t gemm_reserve(hipStream_t s, int m, int kg, int n) {
     return splitk_workspace(s, ints, &err) ? hipSuccess : err;
 }
 
+// The reduction of a.splits slabs in a.ws with the epilogue.
+template <int OUT, bool HAS_BIAS, bool STATIC>
+static hipError_t reduce_splits(hipStream_t s, const GemmArgs& a) {
+    const int64_t mn = (int64_t)a.m * a.n;
+    const uintptr_t need = OUT == OUT_BF16 ? 7u : 15u;
+    const bool vec = (a.n % 4) == 0 && (out_ld(a) % 4) == 0 && (reinterpret_cast<uintptr_t>(a.out) & need) == 0;
+    const int64_t work = vec ? mn / 4 : mn;
+    const unsigned grid = (unsigned)std::min<int64_t>((work + 255) / 256, 256 * 16);
+    if (vec) {
+        switch (a.splits) {
+            case 2: splitk_reduce_kernel<OUT, HAS_BIAS, STATIC, true, 2><<<grid, 256, 0, s>>>(a); break;
+            case 3: splitk_reduce_kernel<OUT, HAS_BIAS, STATIC, true, 3><<<grid, 256, 0, s>>>(a); break;
+            case 4: splitk_reduce_kernel<OUT, HAS_BIAS, STATIC, true, 4><<<grid, 256, 0, s>>>(a); break;
+            default: splitk_reduce_kernel<OUT, HAS_BIAS, STATIC, true><<<grid, 256, 0, s>>>(a); break;
+        }
+    } else {
+        splitk_reduce_kernel<OUT, HAS_BIAS, STATIC, false><<<grid, 256, 0, s>>>(a);
+    }
+    return hipGetLastError();
+}
+
 // Launches the chosen configuration: one kernel, or for S > 1 the split
 // kernel (raw i32 partials) and the reduction that applies the epilogue.
 // ws_fixed: caller-provided slab memory of at least splits*m*n i32 (the
@@ -1192,22 +1265,7 @@ static hipError_t run_gemm(hipStream_t s, bool al, bool dma, const TileChoice& t
     else
         err = go<128, 128, 2, 2, OUT_I32, false, false, true>(s, al, a);
     if (err != hipSuccess) return err;
-    const int64_t mn = (int64_t)a.m * a.n;
-    const uintptr_t need = OUT == OUT_BF16 ? 7u : 15u;
-    const bool vec = (a.n % 4) == 0 && (out_ld(a) % 4) == 0 && (reinterpret_cast<uintptr_t>(a.out) & need) == 0;
-    const int64_t work = vec ? mn / 4 : mn;
-    const unsigned grid = (unsigned)std::min<int64_t>((work + 255) / 256, 256 * 16);
-    if (vec) {
-        switch (a.splits) {
-            case 2: splitk_reduce_kernel<OUT, HAS_BIAS, STATIC, true, 2><<<grid, 256, 0, s>>>(a); break;
-            case 3: splitk_reduce_kernel<OUT, HAS_BIAS, STATIC, true, 3><<<grid, 256, 0, s>>>(a); break;
-            case 4: splitk_reduce_kernel<OUT, HAS_BIAS, STATIC, true, 4><<<grid, 256, 0, s>>>(a); break;
-            default: splitk_reduce_kernel<OUT, HAS_BIAS, STATIC, true><<<grid, 256, 0, s>>>(a); break;
-        }
-    } else {
-        splitk_reduce_kernel<OUT, HAS_BIAS, STATIC, false><<<grid, 256, 0, s>>>(a);
-    }
-    return hipGetLastError();
+    return reduce_splits<OUT, HAS_BIAS, STATIC>(s, a);
 }
 
 // Column split of a 256x256 grid whose last round would run mostly empty
@@ -1240,8 +1298,92 @@ static int column_split(int m, int kg, int n, const TileChoice& tc, bool dma) {
     return cost < 4.0 * (double)rounds ? n_main : 0;
 }
 
+// ---------------------------------------------------------------- padded operands
+// The DMA kernel reads whole 128-byte K stages from 16-byte aligned rows.
+// Operands that are not so (K % 128 != 0, or a pointer off by a word) are
+// first copied to the stream's workspace (slot 1) with their rows zero-padded
+// to a multiple of 128 bytes (the zeros add nothing to an exact integer sum);
+// the copy is one launch over both operands at memory speed, and the GEMM then
+// runs the tiles of an aligned shape. The register-staged kernel instead loads
+// such rows word by word, holds one K stage in flight and has no tile below
+// 128x128, and is the slower one at every size measured (M x K x N, register-
+// staged -> copy + DMA kernel): 40x60x130 10.0 -> 2.6 + 3.4 us, 64x520x1024
+// 24.4 -> 2.9 + 5.2, 2000x132x4000 21.7 -> 3.4 + 11.1, 333x2900x1111 51.6 ->
+// 6.2 + 11.2; 2000x5000x5000 220 -> 90 us for the whole linear.
+// The workspace for it is bounded; larger operands, a stream under capture
+// whose workspace is too small and the no-allocation entry take the
+// register-staged kernel.
+constexpr size_t PAD_MAX_BYTES = size_t(512) << 20;
+
+struct PadShape {
+    int kg, kp;  // words of a row, and of a padded row (a multiple of 4)
+};
+static PadShape pad_shape(int kg, int words) { return {kg, (kg + words - 1) / words * words}; }
+
+__global__ __launch_bounds__(256) void pad_rows_kernel(const uint32_t* x, const uint32_t* w, uint32_t m, PadShape px,
+                                                       PadShape pw, int64_t chunks_x, int64_t chunks, v4i* dst) {
+    typedef int v4iu __attribute__((ext_vector_type(4), aligned(4)));
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < chunks; i += (int64_t)gridDim.x * 256) {
+        const bool isx = i < chunks_x;
+        const int kg = isx ? px.kg : pw.kg, cpr = (isx ? px.kp : pw.kp) >> 2;
+        const int64_t j = isx ? i : i - chunks_x;
+        const int64_t row = chunks < (int64_t(1) << 32) ? (int64_t)((uint32_t)j / (uint32_t)cpr) : j / cpr;
+        const int k = 4 * (int)(j - row * cpr);
+        const uint32_t* src = (isx ? x : w) + row * kg + k;
+        v4i v = {0, 0, 0, 0};
+        if (k + 4 <= kg) {
+            v = *reinterpret_cast<const v4iu*>(src);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 3; ++e)
+                if (k + e < kg) v[e] = (int)src[e];
+        }
+        dst[i] = v;
+    }
+}
+
+// Pads both operands into the stream's workspace; false if that is not to be
+// had (the caller then takes the register-staged kernel), or *err set.
+static bool pad_operands(hipStream_t s, const uint32_t** xq, const uint32_t** wq, int m, int n, PadShape px, PadShape pw,
+                         hipError_t* err) {
+    *err = hipSuccess;
+    const size_t ints = (size_t)m * px.kp + (size_t)n * pw.kp;
+    if (ints * 4 > PAD_MAX_BYTES) return false;
+    int* ws = splitk_workspace(s, ints, err, 1);
+    if (!ws) {
+        if (*err == hipErrorStreamCaptureUnsupported) {
+            (void)hipGetLastError();
+            *err = hipSuccess;
+        } else if (*err == hipSuccess) {
+            *err = hipErrorOutOfMemory;
+        }
+        return false;
+    }
+    const int64_t cx = (int64_t)m * (px.kp / 4), ct = (int64_t)(ints / 4);
+    const unsigned grid = (unsigned)std::min<int64_t>((ct + 255) / 256, 256 * 16);
+    pad_rows_kernel<<<grid, 256, 0, s>>>(*xq, *wq, (uint32_t)m, px, pw, cx, ct, reinterpret_cast<v4i*>(ws));
+    if ((*err = hipGetLastError()) != hipSuccess) return false;
+    *xq = reinterpret_cast<const uint32_t*>(ws);
+    *wq = *xq + (size_t)m * px.kp;
+    return true;
+}
+
+// Workspace elements (slot 1) of the padded operands of a shape: int8 rows
+// (W8A8), or int8 and int4 rows (W4A8); 0 where they are not padded.
+size_t gemm_pad_workspace_ints(int m, int kg, int n) {
+    const PadShape p = pad_shape(kg, 32);
+    const size_t ints = ((size_t)m + n) * p.kp;  // covers W4A8, whose weight rows are half as long
+    return p.kp != kg && ints * 4 <= PAD_MAX_BYTES ? ints : 0;
+}
+
 hipError_t launch_gemm_i8(hipStream_t s, const uint32_t* xq, const uint32_t* wq, const float* sx,
                           const float* sw, const float* bias, void* out, int out_dtype, int m, int kg, int n) {
+    if (kg > 0 && !(gemm_aligned(xq, wq, kg) && (kg * 4) % 128 == 0)) {
+        const PadShape p = pad_shape(kg, 32);
+        hipError_t err;
+        if (pad_operands(s, &xq, &wq, m, n, p, p, &err)) kg = p.kp;
+        else if (err != hipSuccess) return err;
+    }
     GemmArgs a{xq, wq, sx, sw, bias, out, m, kg, n, 0.f, 0.f, 1, nullptr};
     const bool al = gemm_aligned(xq, wq, kg);
     const bool dma = al && ((kg * 4) % 128 == 0);
@@ -1377,28 +1519,16 @@ hipError_t launch_gemm_i8_static(hipStream_t s, const uint32_t* xq, const uint32
 
 // W4A8 prefill GEMM (matmul_q4_dyn, crates/kernels/wgsl/matmul_q4_dyn.wgsl).
 // k is the raw K (k % 8 == 0); the activation keeps its int8 [M, K/4] layout.
-//  - M >= Q4_EXPAND_M and K % 32 == 0: the int4 weights are expanded once to
-//    int8 ([N, K/4], the same values sign-extended) in a per-stream
-//    workspace, and the int8 GEMM runs on them. The accumulators are the same
-//    integers, so the output is bit-identical; the expansion moves 1.5*N*K
-//    bytes, small beside the GEMM at these M.
-//  - otherwise the register-staged kernel with int4 B unpacked on the way
-//    into LDS.
-constexpr int Q4_EXPAND_M = 256;
-
-__global__ __launch_bounds__(256) void expand_q4_kernel(const v4i* w4, v4i* w8, int64_t pieces) {
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < pieces; i += (int64_t)gridDim.x * 256) {
-        v4i lo, hi;
-        unpack_q4x4(w4[i], lo, hi);
-        w8[2 * i] = lo;
-        w8[2 * i + 1] = hi;
-    }
-}
-
-size_t gemm_q4_workspace_ints(int m, int k, int n) {
-    return (m >= Q4_EXPAND_M && k % 32 == 0) ? (size_t)n * (k / 4) : 0;
-}
-
+// K % 128 == 0 and 16-byte aligned operands (or padded to that): the DMA kernel with int4 B, on
+// the tiles of the int8 GEMM in their 128-byte-stage forms. The unpacking (10
+// vector instructions per 32 x 16-byte fragment) runs beside the MFMAs it
+// feeds, and B moves half the bytes. Expanding the weights to int8 in memory
+// first (as from 256 rows before) cost 1.5 N K bytes of traffic on every call:
+// 512x4096x11008 13.6 + 34.9 us -> 39.0; the register-staged kernel, before
+// that the one below 256 rows, has one 128x128 tile shape: whole linears at
+// 64x4096x4096 42 -> 23 us, 128x4096x11008 45 -> 34.
+// Anything else: the register-staged kernel with int4 B unpacked on the way
+// into LDS.
 template <int OUT, bool HAS_BIAS>
 static hipError_t go_q4(hipStream_t s, bool aligned, const GemmArgs& a) {
     TileChoice tc = choose_tiles(a.m, a.kg, a.n);
@@ -1406,22 +1536,58 @@ static hipError_t go_q4(hipStream_t s, bool aligned, const GemmArgs& a) {
     return go<128, 128, 2, 2, OUT, HAS_BIAS, false, false, true>(s, aligned, a);
 }
 
+template <int OUT, bool HAS_BIAS, bool SPLITK>
+static hipError_t go_q4_dma(hipStream_t s, int cfg, const GemmArgs& a) {
+    switch (cfg) {
+        case TILE_256: return go_dma<256, 256, 2, 4, 4, 64, OUT, HAS_BIAS, false, SPLITK, false, true, true>(s, a);
+        case TILE_256x128: return go_dma<256, 128, 4, 2, 3, 128, OUT, HAS_BIAS, false, SPLITK, false, false, true>(s, a);
+        case TILE_128: return go_dma<128, 128, 2, 2, 4, 64, OUT, HAS_BIAS, false, SPLITK, false, false, true>(s, a);
+        case TILE_64x128: return go_dma<64, 128, 2, 2, 4, 128, OUT, HAS_BIAS, false, SPLITK, false, false, true>(s, a);
+        case TILE_32x64:
+            if ((a.kg * 4) % 256 == 0) return go_dma<32, 64, 1, 2, 4, 256, OUT, HAS_BIAS, false, SPLITK, false, false, true>(s, a);
+            [[fallthrough]];
+        default: return go_dma<64, 64, 2, 2, 8, 128, OUT, HAS_BIAS, false, SPLITK, false, false, true>(s, a);
+    }
+}
+
+template <int OUT, bool HAS_BIAS>
+static hipError_t run_q4(hipStream_t s, GemmArgs a) {
+    const TileChoice tc = choose_tiles(a.m, a.kg, a.n);
+    if (tc.splits > 1) {
+        hipError_t err = hipSuccess;
+        a.ws = splitk_workspace(s, (size_t)tc.splits * a.m * a.n, &err);
+        if (a.ws) {
+            a.splits = tc.splits;
+            if ((err = go_q4_dma<OUT_I32, false, true>(s, tc.cfg, a)) != hipSuccess) return err;
+            return reduce_splits<OUT, HAS_BIAS, false>(s, a);
+        }
+        // Capturing without the workspace: the same tiles, unsplit.
+        if (err != hipErrorStreamCaptureUnsupported) return err == hipSuccess ? hipErrorOutOfMemory : err;
+        (void)hipGetLastError();
+    }
+    return go_q4_dma<OUT, HAS_BIAS, false>(s, tc.cfg, a);
+}
+
 hipError_t launch_gemm_q4(hipStream_t s, const uint32_t* xq, const uint32_t* wq, const float* sx,
                           const float* sw, const float* bias, void* out, int out_dtype, int m, int k, int n) {
     // Aligned 16-byte loads need 16-byte rows in both operands: K % 32 == 0.
     const bool al = (k % 32) == 0 && ((reinterpret_cast<uintptr_t>(xq) | reinterpret_cast<uintptr_t>(wq)) & 15u) == 0;
-    const size_t ints = gemm_q4_workspace_ints(m, k, n);
-    if (al && ints) {
-        hipError_t err = hipSuccess;
-        int* w8 = splitk_workspace(s, ints, &err, 1);
-        if (!w8) return err == hipSuccess ? hipErrorOutOfMemory : err;
-        const int64_t pieces = (int64_t)n * k / 32;
-        const unsigned grid = (unsigned)std::min<int64_t>((pieces + 255) / 256, 256 * 8);
-        expand_q4_kernel<<<grid, 256, 0, s>>>(reinterpret_cast<const v4i*>(wq), reinterpret_cast<v4i*>(w8), pieces);
-        if ((err = hipGetLastError()) != hipSuccess) return err;
-        return launch_gemm_i8(s, xq, reinterpret_cast<const uint32_t*>(w8), sx, sw, bias, out, out_dtype, m, k / 4, n);
-    }
     GemmArgs a{xq, wq, sx, sw, bias, out, m, k / 4, n, 0.f, 0.f, 1, nullptr};
+    if (k > 0 && k + 127 < Q4_MAX_K) {
+        bool ready = al && k % 128 == 0;
+        if (!ready) {
+            const PadShape px = pad_shape(k / 4, 32);
+            hipError_t err;
+            ready = pad_operands(s, &a.xq, &a.wq, m, n, px, PadShape{k / 8, px.kp / 2}, &err);
+            if (ready) a.kg = px.kp;
+            else if (err != hipSuccess) return err;
+        }
+        if (ready) switch (out_dtype) {
+            case OUT_I32: return run_q4<OUT_I32, false>(s, a);
+            case OUT_F32: return bias ? run_q4<OUT_F32, true>(s, a) : run_q4<OUT_F32, false>(s, a);
+            default: return bias ? run_q4<OUT_BF16, true>(s, a) : run_q4<OUT_BF16, false>(s, a);
+        }
+    }
     switch (out_dtype) {
         case OUT_I32: return go_q4<OUT_I32, false>(s, al, a);
         case OUT_F32: return bias ? go_q4<OUT_F32, true>(s, al, a) : go_q4<OUT_F32, false>(s, al, a);

@@ -1,0 +1,71 @@
+"""GEMMs whose rows the DMA kernel cannot read as they are (K % 128 != 0, or
+operands off by a word) run on zero-padded copies: accumulators against exact
+int64 sums around the 128-byte stage, for int8 and int4 weights; and a capture
+without a workspace, which takes the other kernel, against the eager bits."""
+import numpy as np
+import pytest
+import torch
+
+from brain_amd import ops
+from oracle import oracle as o
+
+pytestmark = pytest.mark.gpu
+
+
+def words(rng, rows, kw):
+    return torch.from_numpy(rng.integers(-2 ** 31, 2 ** 31, (rows, kw), dtype=np.int64).astype(np.int32)).cuda()
+
+
+def int8_of(t):
+    return t.contiguous().cpu().numpy().view(np.int8).astype(np.int64)
+
+
+def int4_of(t):
+    w = t.cpu().numpy().view(np.uint32)
+    n = np.stack([(w >> (4 * b)) & 15 for b in range(8)], -1).reshape(w.shape[0], -1).astype(np.int64)
+    return np.where(n > 7, n - 16, n)
+
+
+@pytest.mark.parametrize("m,k,n", [(33, 4, 1), (33, 124, 65), (64, 128, 64), (65, 132, 130), (200, 1000, 257),
+                                   (333, 2900, 111), (40, 6148, 70), (300, 516, 1030)])
+@pytest.mark.parametrize("off", [0, 1])
+def test_padded_i8_accumulators(gpu, m, k, n, off):
+    rng = np.random.default_rng(m + k + n)
+    x = words(rng, 1, m * k // 4 + off).view(-1)[off:].view(m, k // 4)  # off: not 16-byte aligned
+    w = words(rng, n, k // 4)
+    one = torch.ones(max(m, n), device="cuda")
+    got = ops.matmul_i8(x, w, one[:m], one[:n], None, torch.int32, "dyn").cpu().numpy()
+    assert np.array_equal(got, int8_of(x) @ int8_of(w).T)
+
+
+@pytest.mark.parametrize("m,k,n", [(33, 8, 1), (33, 120, 65), (64, 128, 64), (65, 136, 130), (200, 1000, 257),
+                                   (512, 2048, 300), (300, 6976, 70), (40, 4096, 129), (1030, 256, 520)])
+def test_q4_accumulators(gpu, m, k, n):
+    rng = np.random.default_rng(m + k + n + 7)
+    x, w = words(rng, m, k // 4), words(rng, n, k // 8)
+    one = torch.ones(max(m, n), device="cuda")
+    got = ops.matmul_q4(x, w, one[:m], one[:n], None, torch.int32, "dyn").cpu().numpy()
+    assert np.array_equal(got, int8_of(x) @ int4_of(w).T)
+
+
+@pytest.mark.parametrize("reserve", [False, True])
+@pytest.mark.parametrize("q4", [False, True])
+def test_ragged_capture(gpu, q4, reserve):
+    m, k, n = 150, 1000, 420
+    rng = np.random.default_rng(5)
+    x, w = words(rng, m, k // 4), words(rng, n, k // (8 if q4 else 4))
+    sx, sw = torch.rand(m, device="cuda"), torch.rand(n, device="cuda")
+    mm = ops.matmul_q4 if q4 else ops.matmul_i8
+    eager = mm(x, w, sx, sw, None, torch.float32, "dyn").clone()
+    out = torch.empty(m, n, device="cuda")
+    cap = torch.cuda.Stream()
+    if reserve:
+        ops.reserve_workspace(m, k, n, cap)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=cap):
+        mm(x, w, sx, sw, None, torch.float32, "dyn", out=out)
+    for _ in range(3):
+        out.fill_(0)
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
