@@ -11,8 +11,15 @@ from ._lib import BH_OUT_BF16, BH_OUT_F32, BH_OUT_I32, check, load
 _CODES = {torch.float32: BH_OUT_F32, torch.bfloat16: BH_OUT_BF16, torch.int32: BH_OUT_I32}
 
 
-def _stream():
-    return torch.cuda.current_stream().cuda_stream
+# The handle of the current device's current stream. The public call builds a
+# Stream object on the way (3.4 us, a third of a decode linear's host time;
+# this one 0.1 us).
+if hasattr(torch._C, "_cuda_getCurrentRawStream"):
+    def _stream():
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+else:
+    def _stream():
+        return torch.cuda.current_stream().cuda_stream
 
 
 def _ptr(t):
@@ -156,15 +163,21 @@ def linear_i8(x, wq, sw, bias=None, out_dtype=torch.float32, sx=None, xq=None, o
         _need(bias, torch.float32, n, "bias")
     if out_dtype not in (torch.float32, torch.bfloat16):
         raise ValueError(f"linear_i8: out_dtype {out_dtype}, expected float32 or bfloat16")
-    sx = torch.empty(m, device=x.device, dtype=torch.float32) if sx is None else sx
-    xq = torch.empty(m, k // 4, device=x.device, dtype=torch.int32) if xq is None else xq
-    _need(sx, torch.float32, m, "sx")
-    _need(xq, torch.int32, m * (k // 4), "xq")
-    code = {torch.float32: BH_OUT_F32, torch.bfloat16: BH_OUT_BF16}[out_dtype]
+    if sx is None and xq is None:  # one allocation for both: [m, k/4] codes, then [m] scales
+        scratch = torch.empty(m * (k // 4) + m, device=x.device, dtype=torch.int32)
+        xq_ptr = scratch.data_ptr()
+        sx_ptr = xq_ptr + m * k
+    else:
+        sx = torch.empty(m, device=x.device, dtype=torch.float32) if sx is None else sx
+        xq = torch.empty(m, k // 4, device=x.device, dtype=torch.int32) if xq is None else xq
+        _need(sx, torch.float32, m, "sx")
+        _need(xq, torch.int32, m * (k // 4), "xq")
+        sx_ptr, xq_ptr = sx.data_ptr(), xq.data_ptr()
+    code = BH_OUT_F32 if out_dtype == torch.float32 else BH_OUT_BF16
     out = torch.empty(m, n, device=x.device, dtype=out_dtype) if out is None else out
     _need(out, out_dtype, m * n, "out")
-    check(load().bh_linear_i8(_stream(), _ptr(x), _ptr(wq), _ptr(sw), _ptr(bias), _ptr(sx), _ptr(xq),
-                              _ptr(out), code, m, k, n))
+    check(load().bh_linear_i8(_stream(), _ptr(x), _ptr(wq), _ptr(sw), _ptr(bias), sx_ptr, xq_ptr, _ptr(out), code, m, k,
+                              n))
     return out
 
 
