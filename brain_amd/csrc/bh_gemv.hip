@@ -1195,6 +1195,63 @@ hipError_t launch_gemv_i8(hipStream_t s, const uint32_t* xq, const uint32_t* wq,
     return gv_out<2>(s, aligned, out_dtype, a);
 }
 
+// K split over workgroups: the raw i32 sums of K quarter p go to
+// parts[p][m][n], for a consumer that reads the projection anyway and adds the
+// four (exact in any order) and applies the epilogue itself. For narrow N over
+// a long K, where one workgroup per 16 columns leaves three quarters of the
+// chip idle and each one streams the whole K (the decoder's output and down
+// projections: 64 workgroups of 32-48 KB of weights, bound by what one CU
+// draws). Batch-8 decode at 128-192
+// positions: output projection 4.2 -> 2.5 us, down projection 5.2 -> 2.5 us (the
+// norms that add the sums 3.1 -> 3.0 us), the step 1.06 -> 0.98 ms.
+constexpr int GEMV_PARTS = 4;
+template <int CPW>
+__global__ __launch_bounds__(256) void gemv_i8_part_kernel(const uint8_t* xq, const uint8_t* wq, int m, int kbytes,
+                                                           int n, int* parts) {
+    __shared__ int red[4][4][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int col = blockIdx.x * 16 + (lane & 15);
+    const int k0 = (blockIdx.y * 4 + wave) * CPW * 64 + (lane >> 4) * 16;
+    const uint8_t* wp = wq + (int64_t)col * kbytes + k0;
+    const uint8_t* xp = xq + (int64_t)min(lane & 15, m - 1) * kbytes + k0;  // rows past m are not stored
+    v4i w[CPW], x[CPW];
+#pragma unroll
+    for (int u = 0; u < CPW; ++u) w[u] = *reinterpret_cast<const v4i*>(wp + 64 * u);
+#pragma unroll
+    for (int u = 0; u < CPW; ++u) x[u] = *reinterpret_cast<const v4i*>(xp + 64 * u);
+    v4i acc = {0, 0, 0, 0};
+#pragma unroll
+    for (int u = 0; u < CPW; ++u) acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[u], w[u], acc, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) red[wave][i][lane] = acc[i];
+    __syncthreads();
+    const int row = 4 * (lane >> 4) + wave;  // wave i adds up register i of the four waves
+    int s = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) s += red[q][wave][lane];
+    if (row < m) parts[((int64_t)blockIdx.y * m + row) * n + col] = s;
+}
+
+// Whether launch_gemv_i8_parts takes a shape: at most 16 rows, whole K chunks
+// per wave, and few enough column groups that the split fills idle CUs.
+bool gemv_parts_ok(int m, int kg, int n) {
+    const int chunks = kg * 4 / 64;
+    return m >= 1 && m <= 16 && kg % 16 == 0 && chunks % 16 == 0 && chunks >= 32 && chunks <= 64 && n % 16 == 0 &&
+           n / 16 <= 128;
+}
+// xq and wq 16-byte aligned; parts [4][m][n].
+hipError_t launch_gemv_i8_parts(hipStream_t s, const uint32_t* xq, const uint32_t* wq, int* parts, int m, int kg, int n) {
+    const dim3 grid(n / 16, GEMV_PARTS);
+    const uint8_t *x = reinterpret_cast<const uint8_t*>(xq), *w = reinterpret_cast<const uint8_t*>(wq);
+    switch (kg * 4 / 1024) {
+        case 2: gemv_i8_part_kernel<2><<<grid, 256, 0, s>>>(x, w, m, kg * 4, n, parts); break;
+        case 3: gemv_i8_part_kernel<3><<<grid, 256, 0, s>>>(x, w, m, kg * 4, n, parts); break;
+        case 4: gemv_i8_part_kernel<4><<<grid, 256, 0, s>>>(x, w, m, kg * 4, n, parts); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
 hipError_t launch_gemv_i8_gated(hipStream_t s, const uint32_t* xq, const uint32_t* wq, const float* sx,
                                 const float* sw, const float* gate, int gate_stride, int gate_col, float* out, int m,
                                 int kg, int n) {

@@ -54,6 +54,8 @@ hipError_t launch_gemv_i8(hipStream_t s, const uint32_t* xq, const uint32_t* wq,
                           const float* sw, const float* bias, void* out, int out_dtype, int m, int kg, int n,
                           bool keep_cached = false, float* am_v = nullptr, uint32_t* am_i = nullptr,
                           uint32_t* am_n = nullptr, int am_stride = 0);
+bool gemv_parts_ok(int m, int kg, int n);
+hipError_t launch_gemv_i8_parts(hipStream_t s, const uint32_t* xq, const uint32_t* wq, int* parts, int m, int kg, int n);
 hipError_t gemm_reserve(hipStream_t s, int m, int kg, int n);
 hipError_t launch_gemm_i8(hipStream_t s, const uint32_t* xq, const uint32_t* wq, const float* sx,
                           const float* sw, const float* bias, void* out, int out_dtype, int m, int kg, int n);
@@ -144,11 +146,17 @@ struct NormQuantArgs {
     float* sx;             // [rows]
     uint32_t* xq;          // [rows, xq_words]
     int xq_words;
+    // PARTS: b is the projection in four raw i32 sums [4][rows][d] (row_map
+    // null) with the scales of its epilogue: sx (read before this kernel
+    // writes it, by the same workgroup) and bsw [d].
+    const int* parts = nullptr;
+    const float* bsw = nullptr;
+    int rows = 0;
 };
 
 // rmsnorm_rows.wgsl:24-44 (y = x * (1/sqrt(mean(x^2) + eps)) * w) on x = a + b
 // (add2.wgsl) or an embedding row (embed.wgsl), then the row's int8 quant.
-template <int G>
+template <int G, bool PARTS = false>
 __global__ __launch_bounds__(RT) void norm_quant_kernel(NormQuantArgs p) {
     __shared__ float red[RT / 64];
     const int r = blockIdx.x;
@@ -165,13 +173,33 @@ __global__ __launch_bounds__(RT) void norm_quant_kernel(NormQuantArgs p) {
     for (int g = 0; g < G; ++g) wv[g] = w4[min((int)threadIdx.x + g * RT, d4 - 1)];
     float4 x[G];
     float ss = 0.0f;
+    int4 pt[PARTS ? G : 1][4];
+    float4 psw[PARTS ? G : 1];
+    float psx = 0.0f;
+    if constexpr (PARTS) {
+        psx = p.sx[r];
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const int i = min((int)threadIdx.x + g * RT, d4 - 1);
+            psw[g] = reinterpret_cast<const float4*>(p.bsw)[i];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) pt[g][q] = reinterpret_cast<const int4*>(p.parts)[((size_t)q * p.rows + r) * d4 + i];
+        }
+    }
 #pragma unroll
     for (int g = 0; g < G; ++g) {
         const int i = threadIdx.x + g * RT;
         x[g] = make_float4(0.f, 0.f, 0.f, 0.f);
         if (i < d4) {
             float4 v = src[i];
-            if (add) v = add4(v, add[i]);
+            if constexpr (PARTS) {
+                auto sum = [&](int4 a, int4 b, int4 c, int4 d) {
+                    return make_int4(a.x + b.x + c.x + d.x, a.y + b.y + c.y + d.y, a.z + b.z + c.z + d.z, a.w + b.w + c.w + d.w);
+                };
+                const int4 a = sum(pt[g][0], pt[g][1], pt[g][2], pt[g][3]);
+                v = add4(v, make_float4(dequant(a.x, psx, psw[g].x), dequant(a.y, psx, psw[g].y),
+                                        dequant(a.z, psx, psw[g].z), dequant(a.w, psx, psw[g].w)));
+            } else if (add) v = add4(v, add[i]);
             x[g] = v;
             ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
         }
@@ -1003,6 +1031,7 @@ struct bh_qwen3 {
 
     float *res = nullptr, *res2 = nullptr, *qkv = nullptr, *q = nullptr, *proj = nullptr, *gu = nullptr;
     float *part_o = nullptr, *part_ml = nullptr;  // attention chunk partials
+    int* parts = nullptr;                         // K-quarter sums of a projection [4][rows <= 16][d_model]
     uint32_t max_splits = 0;
     bool flash = false;  // prompt attention on launch_flash_prefill (else attn_split + merge)
     const uint32_t* cur_pos = nullptr;
@@ -1098,7 +1127,10 @@ int launch_linear(bh_qwen3* e, const uint32_t* w, const float* sw, float* out, i
 
 int launch_norm_quant(bh_qwen3* e, const NormQuantArgs& a, int rows) {
     const int groups = (a.d / 4 + RT - 1) / RT;
-    if (groups <= 1) norm_quant_kernel<1><<<rows, RT, 0, e->stream>>>(a);
+    if (a.parts) {
+        if (groups <= 1) norm_quant_kernel<1, true><<<rows, RT, 0, e->stream>>>(a);
+        else norm_quant_kernel<2, true><<<rows, RT, 0, e->stream>>>(a);
+    } else if (groups <= 1) norm_quant_kernel<1><<<rows, RT, 0, e->stream>>>(a);
     else if (groups <= 2) norm_quant_kernel<2><<<rows, RT, 0, e->stream>>>(a);
     else if (groups <= 4) norm_quant_kernel<4><<<rows, RT, 0, e->stream>>>(a);
     else norm_quant_kernel<8><<<rows, RT, 0, e->stream>>>(a);
@@ -1189,6 +1221,7 @@ int run_rows(bh_qwen3* e, int rows, const uint32_t* tok, const uint32_t* pos, co
     const float scale = 1.0f / sqrtf((float)hd);
     // Prompt rows: whole runs of consecutive positions, one per sequence.
     const bool flash = !decode && rows_per_seq > 0 && rows % rows_per_seq == 0 && e->flash;
+    bool last_parts = false;  // the last down projection is in e->parts
     for (uint32_t l = 0; l < c.n_layers; ++l) {
         const bh_qwen3::Layer& Ly = e->L[l];
         void* kc = static_cast<uint8_t*>(e->kc) + l * e->layer_kv * e->kv_elem;
@@ -1196,12 +1229,24 @@ int run_rows(bh_qwen3* e, int rows, const uint32_t* tok, const uint32_t* pos, co
         const size_t lsc = (size_t)l * e->slots * nkv;
         float* ksl = e->c.kv_int8 ? e->kscale + lsc : nullptr;
         float* vsl = e->c.kv_int8 ? e->vscale + lsc : nullptr;
+        // Decode rows whose norm is a launch of its own: the output and down
+        // projections leave raw K-quarter sums for that norm to add.
+        auto parts_of = [&](int k) {
+            return decode && !e->nofuse && e->parts && d <= 2 * 4 * RT && rows <= 16 && gemv_parts_ok(rows, k / 4, d) &&
+                   !tuned_variant((uint32_t)rows, (uint32_t)d, (uint32_t)k);
+        };
+        auto add_parts = [&](NormQuantArgs& n, const float* sw) {
+            n.parts = e->parts;
+            n.bsw = sw;
+            n.rows = rows;
+        };
         // Residual stream ping-pongs between res and res2 (two swaps per
         // layer): a fused producer's workgroup 0 writes the new residual while
         // other workgroups still read the old one.
         const bool fuse = !e->nofuse && fused_ok(rows, d, (int)e->W, fuse_norm_rows()) &&
                           fused_ok(rows, d, 2 * ff, fuse_norm_rows());
         const bool fuse_sw = !e->nofuse && ff % 64 == 0 && fused_ok(rows, ff, d, fuse_swiglu_rows());
+        const bool oparts = !fuse && parts_of((int)e->hq), dparts = !fuse && !fuse_sw && parts_of(ff);
         if (fuse) {
             BH_HIP(launch_gemv_i8_pre(e->stream, 3, l == 0 ? tok : nullptr, e->emb, l == 0 ? nullptr : cur,
                                       l == 0 ? nullptr : e->proj, Ly.ln1, nxt, c.rms_eps, Ly.wqkv, Ly.sqkv, e->qkv,
@@ -1215,6 +1260,7 @@ int run_rows(bh_qwen3* e, int rows, const uint32_t* tok, const uint32_t* pos, co
             } else {
                 na.a = cur;
                 na.b = e->proj;  // previous layer's down projection
+                if (dparts) add_parts(na, e->L[l - 1].sdown);
             }
             na.res_out = nxt;
             na.w = Ly.ln1;
@@ -1276,7 +1322,8 @@ int run_rows(bh_qwen3* e, int rows, const uint32_t* tok, const uint32_t* pos, co
         } else {
             if (flash) BH_HIP(launch_quantize_rows(e->stream, e->q, rows, (int)e->hq, e->sx, e->xq), "context quantization");
             else BH_TRY(launch_combine_quant(e, rows, splits));
-            BH_TRY(launch_linear(e, Ly.wo, Ly.so, e->proj, rows, (int)e->hq, d));
+            if (oparts) BH_HIP(launch_gemv_i8_parts(e->stream, e->xq, Ly.wo, e->parts, rows, (int)e->hq / 4, d), "output projection launch");
+            else BH_TRY(launch_linear(e, Ly.wo, Ly.so, e->proj, rows, (int)e->hq, d));
         }
         if (fuse) {
             BH_HIP(launch_gemv_i8_pre(e->stream, 3, nullptr, nullptr, cur, e->proj, Ly.ln2, nxt, c.rms_eps, Ly.wgu,
@@ -1294,6 +1341,7 @@ int run_rows(bh_qwen3* e, int rows, const uint32_t* tok, const uint32_t* pos, co
             nb.sx = e->sx;
             nb.xq = e->xq;
             nb.xq_words = d / 4;
+            if (oparts) add_parts(nb, Ly.so);
             BH_TRY(launch_norm_quant(e, nb, rows));
             std::swap(cur, nxt);
             BH_TRY(launch_linear(e, Ly.wgu, Ly.sgu, e->gu, rows, d, 2 * ff));
@@ -1304,8 +1352,10 @@ int run_rows(bh_qwen3* e, int rows, const uint32_t* tok, const uint32_t* pos, co
                    "fused swiglu + down launch");
         } else {
             BH_TRY(launch_swiglu_quant(e, rows));
-            BH_TRY(launch_linear(e, Ly.wdown, Ly.sdown, e->proj, rows, ff, d));
+            if (dparts) BH_HIP(launch_gemv_i8_parts(e->stream, e->xq, Ly.wdown, e->parts, rows, ff / 4, d), "down projection launch");
+            else BH_TRY(launch_linear(e, Ly.wdown, Ly.sdown, e->proj, rows, ff, d));
         }
+        last_parts = dparts;
     }
     if (n_out <= 0) return BH_OK;
     NormQuantArgs nf{};
@@ -1318,6 +1368,11 @@ int run_rows(bh_qwen3* e, int rows, const uint32_t* tok, const uint32_t* pos, co
     nf.sx = e->sx;
     nf.xq = e->xq;
     nf.xq_words = d / 4;
+    if (last_parts) {  // decode: every row, in order
+        nf.parts = e->parts;
+        nf.bsw = e->L[c.n_layers - 1].sdown;
+        nf.rows = rows;
+    }
     BH_TRY(launch_norm_quant(e, nf, n_out));
     // The head's weights are re-read every step and fit the Infinity Cache
     // (measured: batch-1 step 0.861 ms with ordinary loads, 0.863-0.864 with
@@ -1550,7 +1605,8 @@ int bh_qwen3_create(const bh_qwen3_config* cfg, uint32_t max_batch, uint32_t max
         (rc = dalloc(e, &e->rope_cs, (uint64_t)max_seq * (c.head_dim / 2))) ||
         (rc = dalloc(e, &e->res, R * d)) || (rc = dalloc(e, &e->res2, R * d)) || (rc = dalloc(e, &e->qkv, R * e->W)) || (rc = dalloc(e, &e->q, R * hq)) ||
         (rc = dalloc(e, &e->part_o, PR * c.n_heads * e->max_splits * c.head_dim)) ||
-        (rc = dalloc(e, &e->part_ml, PR * c.n_heads * e->max_splits * 2)) || (rc = dalloc(e, &e->proj, R * d)) || (rc = dalloc(e, &e->gu, R * 2 * ff)) ||
+        (rc = dalloc(e, &e->part_ml, PR * c.n_heads * e->max_splits * 2)) || (rc = dalloc(e, &e->proj, R * d)) ||
+        (rc = dalloc(e, &e->parts, 4 * (uint64_t)std::min<uint32_t>(max_batch, 16) * d)) || (rc = dalloc(e, &e->gu, R * 2 * ff)) ||
         (rc = dalloc(e, &e->sx, R)) || (rc = dalloc(e, &e->xq, R * e->xq_words)) ||
         (rc = dalloc(e, &e->logits, (uint64_t)max_batch * c.vocab)) || (rc = dalloc(e, &e->tmpw, e->tmpw_floats)) ||
         (rc = dalloc(e, &e->am_v, (uint64_t)max_batch * AM_PARTS)) || (rc = dalloc(e, &e->am_i, (uint64_t)max_batch * AM_PARTS)) ||
