@@ -17,7 +17,10 @@
 //                   combine per row that also quantizes the context
 //                   (paged_decode_scores_wg / decode_softmax_batched /
 //                   paged_decode_apply_batched + max_abs_row/quant_pack)
-//   linear o
+//                   Prompt rows with head_dim 64 or 128 take the flash
+//                   kernel (bh_flash.hip) and a row quantization instead.
+//   linear o        (decode, 5 to 16 rows: left as K-quarter sums that the
+//                   next norm_quant adds; the down projection likewise)
 //   norm_quant      residual add + RMSNorm + quant
 //   linear gate|up  stacked like qkv
 //   swiglu_quant    silu(g)*u (silu_mul.wgsl) + quant
