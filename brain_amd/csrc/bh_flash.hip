@@ -21,7 +21,10 @@
 // softmax); at the end the KS parts are merged through LDS in a fixed order.
 // The tiles start at multiples of 32 positions and a masked tile leaves a
 // vector's state as it is, so a row's numbers do not depend on the rows it
-// shares a launch with: any chunking of a prompt gives the same bits.
+// shares a launch with: any chunking of a prompt gives the same bits. (Where
+// an infinity, a NaN or an overflow makes a vector's result not finite, the
+// vector is computed once more by plain_row; which vectors of a shared tile a
+// NaN value reaches does depend on the chunking, and those agree to rounding.)
 //
 // Scores are computed transposed (keys x queries): a lane then holds 16 keys
 // of one query, the softmax statistics need one exchange with lane ^ 32, and
@@ -64,7 +67,7 @@ __device__ __forceinline__ uint32_t hi16x2(float lo, float hi) {
 __device__ __forceinline__ float below_bf16(float x) { return x - bitsf(fbits(x) & 0xffff0000u); }
 
 // Eight floats as three bf16 fragments. (A non-finite operand leaves NaN in
-// the second part: its products are NaN.)
+// the second part and in every result it enters: plain_row takes those.)
 __device__ __forceinline__ void split8(const float (&x)[8], v4i& a, v4i& b, v4i& c) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -113,6 +116,59 @@ struct FlashCfg {
     static_assert(NKC * NT * 8 == KEYS * HD && (VB <= NT || NVB * NT == VB), "whole pieces per thread");
     static_assert(MERGE <= LDS, "the merge fits the tiles' LDS");
 };
+
+// One query vector by one wave in plain f32 over its visible keys alone, for
+// the vectors whose result above is not finite: an infinity times a zero part
+// or a zero weight is NaN there, a NaN value reaches the rows before it in a
+// shared tile, a value that rounds to an infinity in bf16 is lost, and scores
+// below NO_REF leave no weight at all. Here each of them is what the formula
+// gives. Loads are uncoalesced (a lane reads its key's row): this runs for
+// such vectors only.
+template <bool KV8, int HD>
+__device__ void plain_row(const FlashArgs& p, const uint32_t* tslot, int r, int kh, int h, int lane) {
+    float* q = p.q + (size_t)r * p.hq + (size_t)h * HD;
+    const int pos = (int)p.pos[r];
+    using Elem = std::conditional_t<KV8, int8_t, float>;
+    auto row_of = [&](int j) -> size_t { return (size_t)tslot[j >> 5] + (j & 31); };
+    auto score = [&](int j) -> float {
+        const size_t slot = row_of(j);
+        const Elem* k = static_cast<const Elem*>(p.kc) + slot * p.hkv + (size_t)kh * HD;
+        float acc = 0.0f;
+#pragma unroll 4
+        for (int d = 0; d < HD; ++d) acc = acc + q[d] * (float)k[d];
+        if constexpr (KV8) acc = acc * p.ks[slot * p.nkv + kh];
+        return acc * p.scale;
+    };
+    float mx = -INFINITY;
+    for (int j = lane; j <= pos; j += 64) mx = fmaxf(mx, score(j));
+    mx = xor_max<32>(mx);
+    float l = 0.0f, ctx[HD / 64];
+#pragma unroll
+    for (int u = 0; u < HD / 64; ++u) ctx[u] = 0.0f;
+    for (int j0 = 0; j0 <= pos; j0 += 64) {
+        float w = 0.0f;
+        if (j0 + lane <= pos) {
+            const float s = score(j0 + lane);
+            w = s == -INFINITY ? 0.0f : expf(s - mx);
+        }
+        l = l + w;
+        const int n = min(64, pos + 1 - j0);
+        for (int k = 0; k < n; ++k) {
+            const float wk = __shfl(w, k, 64);
+            const size_t slot = row_of(j0 + k);
+            const Elem* v = static_cast<const Elem*>(p.vc) + slot * p.hkv + (size_t)kh * HD;
+#pragma unroll
+            for (int u = 0; u < HD / 64; ++u) {
+                float t = wk * (float)v[lane + 64 * u];
+                if constexpr (KV8) t = t * p.vs[slot * p.nkv + kh];
+                ctx[u] = ctx[u] + t;
+            }
+        }
+    }
+    l = xor_sum<32>(l);
+#pragma unroll
+    for (int u = 0; u < HD / 64; ++u) q[lane + 64 * u] = ctx[u] / l;
+}
 
 template <bool KV8, int HD, int QG, int KS>
 __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p) {
@@ -501,14 +557,29 @@ __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p)
     }
     if (ks == 0) {
         const float inv = 1.0f / (l + xor_lane<32>(l));
-        if (qlive) {
+        float z = 0.0f;  // NaN once a context element is not finite
+#pragma unroll
+        for (int j = 0; j < HD / 32; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                o[j][e] = o[j][e] * inv;
+                z = __builtin_fmaf(o[j][e], 0.0f, z);
+            }
+        const unsigned long long bad = __ballot(qlive && z != 0.0f);
+        uint32_t redo = (uint32_t)bad | (uint32_t)(bad >> 32);  // by col: a vector's two halves
+        if (qlive && !((redo >> col) & 1u)) {
 #pragma unroll
             for (int j = 0; j < HD / 32; ++j)
 #pragma unroll
                 for (int e4 = 0; e4 < 4; ++e4)
                     *reinterpret_cast<float4*>(qrow + 32 * j + 8 * e4 + 4 * half) =
-                        make_float4(o[j][4 * e4] * inv, o[j][4 * e4 + 1] * inv, o[j][4 * e4 + 2] * inv,
-                                    o[j][4 * e4 + 3] * inv);
+                        make_float4(o[j][4 * e4], o[j][4 * e4 + 1], o[j][4 * e4 + 2], o[j][4 * e4 + 3]);
+        }
+        // Live columns only (bad is 0 elsewhere); their queries are not yet
+        // overwritten.
+        for (; redo; redo &= redo - 1u) {
+            const int c = __ffs(redo) - 1, i = qg * RW + c / G;
+            plain_row<KV8, HD>(p, tslot, r0 + i, kh, kh * G + c % G, lane);
         }
     }
 }

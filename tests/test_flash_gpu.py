@@ -119,3 +119,58 @@ def test_flash_prefill_chunking_gives_the_same_bits(gpu, kv8, hd, group):
     cuts = [0, 1, 2, 35, 64, 191, 300]
     parts = torch.cat([s.run(a, b) for a, b in zip(cuts, cuts[1:])], 1)
     assert torch.equal(whole, parts)
+
+
+def plain64(s, p1):
+    """Context of rows 0..p1 in numpy float64, each row over its visible keys alone."""
+    q, kc, vc, slot = (t.cpu().numpy() for t in (s.q, s.k, s.v, s.slot))
+    out = np.empty((s.nseq, p1, s.nh, s.hd))
+    with np.errstate(all="ignore"):
+        for b in range(s.nseq):
+            k, v = (x[slot[b]].reshape(-1, s.nkv, s.hd).astype(np.float64) for x in (kc, vc))
+            if s.kv8:
+                k, v = (x * sc.cpu().numpy()[slot[b]][:, :, None].astype(np.float64) for x, sc in ((k, s.ks), (v, s.vs)))
+            for i in range(p1):
+                for h in range(s.nh):
+                    sc = (q[b, i, h].astype(np.float64) * k[: i + 1, h // s.group]).sum(1) * s.hd ** -0.5
+                    w = np.exp(sc - np.fmax.reduce(sc))
+                    out[b, i, h] = (w[:, None] * v[: i + 1, h // s.group]).sum(0) / w.sum()
+    return out
+
+
+@pytest.mark.parametrize("hd,group", [(128, 2), (64, 3)])
+@pytest.mark.parametrize("what", ["v_nan", "v_inf", "v_top", "k_low", "k_nan", "vs_inf", "ks_nan"])
+def test_flash_prefill_values_at_the_ends_of_f32(gpu, what, hd, group):
+    """A value that is not finite, or rounds to an infinity in bf16, or scores
+    far below any other key, in one cache slot: rows before it do not see it
+    (a masked key is left out, not weighted with zero), rows from it on are
+    what the formula gives, and neither depends on the chunking. The 2-norm
+    bar is the one of the finite cases."""
+    kv8 = what in ("vs_inf", "ks_nan")
+    s = Setup(2, 75, 2, group, hd, kv8, True, seed=21)
+    at = s.slot[0, 0 if what == "k_low" else 37]
+    if what == "v_nan":
+        s.v[at, 5] = float("nan")
+    elif what == "v_inf":
+        s.v[at, 5] = float("inf")
+    elif what == "v_top":
+        s.v[at, 5] = torch.finfo(torch.float32).max
+    elif what == "k_nan":
+        s.k[at, 5] = float("nan")
+    elif what == "k_low":  # row 0 sees this key alone; its score is finite and below -1e34
+        s.q.abs_()
+        s.k[at] = -1e36
+    elif what == "vs_inf":
+        s.vs[at, 0] = float("inf")
+        s.v[at] = torch.where(s.v[at] == 0, torch.ones_like(s.v[at]), s.v[at])  # no 0 x infinity in the formula
+    else:
+        s.ks[at, 0] = float("nan")
+    want = plain64(s, 75)
+    for cuts in ([0, 75], [0, 20, 38, 39, 64, 75]):
+        got = torch.cat([s.run(a, b) for a, b in zip(cuts, cuts[1:])], 1).double().cpu().numpy()
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+        fin = np.isfinite(want)
+        assert np.array_equal(got[~fin & ~np.isnan(want)], want[~fin & ~np.isnan(want)])
+        scale = np.where(fin, np.abs(want), 0).max((0, 1, 2))  # one column holds numbers of another size
+        err = np.abs(np.where(fin, got, 0) - np.where(fin, want, 0))
+        assert (err <= 1e-5 * np.maximum(scale, 1)).all()
