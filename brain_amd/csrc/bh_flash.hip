@@ -6,12 +6,15 @@
 // paged_decode_apply_batched, and the i8 pair of them over an int8 cache:
 // score = (q . code) * kscale * scale, context += (p * code) * vscale). Here
 // an f32 operand x is the exact sum of three bf16 numbers, x = x1 + x2 + x3
-// (8 + 8 + 8 significant bits, each the truncation of what the ones before it
-// leave), and a product of two such operands is the six partial products
-// x1y1, x1y2, x2y1, x2y2, x1y3, x3y1, accumulated in f32 by
-// v_mfma_f32_32x32x16_bf16. The three left out are below 2^-23 of the product,
-// the weight of one rounding in f32. Codes of the int8 cache are exact in one
-// bf16, so a product with them is three partial products.
+// (8 significant bits each, each the rounding to nearest of what the ones
+// before it leave: |x2| <= 2^-8 |x|, |x3| <= 2^-17 |x|), and a product of two
+// such operands is the six partial products x1y1, x1y2, x2y1, x2y2, x1y3,
+// x3y1, accumulated in f32 by v_mfma_f32_32x32x16_bf16. The three left out,
+// x2y3 + x3y2 + x3y3, are at most 2^-24 of the product, the error of one f32
+// multiplication, with either sign; for normal operands 0.06 x 2^-24 on
+// average, where the f32 multiplication's is 0.36 x 2^-24. (Truncated parts
+// leave out up to 8 x 2^-24, always towards zero.) Codes of the int8 cache are
+// exact in one bf16, so a product with them is three partial products.
 // f32 MFMA would take 64 cycles per 2048 multiply-adds, against 6 x 32 cycles
 // per 16384 here (3 x 32 with an int8 cache).
 //
@@ -45,7 +48,7 @@
 // against 164 / 51 us at 2 x 4, and 12 against 17 us at 64 tokens. KS is part
 // of the result's summation order, so it is one per cache type and not chosen
 // by length. Against 64-bit attention, one 2000-token prompt of normal q, k, v:
-// 1.6e-7 (f32 cache) and 3.0e-7 (int8) in the 2-norm; the f32 kernel 2.2e-7
+// 1.4e-7 (f32 cache) and 3.0e-7 (int8) in the 2-norm; the f32 kernel 2.2e-7
 // and 3.3e-7.
 #include <type_traits>
 
@@ -60,11 +63,10 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 
 __device__ __forceinline__ uint32_t fbits(float f) { return __builtin_bit_cast(uint32_t, f); }
 __device__ __forceinline__ float bitsf(uint32_t u) { return __builtin_bit_cast(float, u); }
-// The upper halves of two floats: their truncations to bf16, packed.
+// The upper halves of two floats that are exact in bf16, packed.
 __device__ __forceinline__ uint32_t hi16x2(float lo, float hi) {
     return __builtin_amdgcn_perm(fbits(hi), fbits(lo), 0x07060302u);
 }
-__device__ __forceinline__ float below_bf16(float x) { return x - bitsf(fbits(x) & 0xffff0000u); }
 
 // Eight floats as three bf16 fragments. (A non-finite operand leaves NaN in
 // the second part and in every result it enters: plain_row takes those.)
@@ -72,10 +74,12 @@ __device__ __forceinline__ void split8(const float (&x)[8], v4i& a, v4i& b, v4i&
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const float x0 = x[2 * i], x1 = x[2 * i + 1];
-        a[i] = (int)hi16x2(x0, x1);
-        const float r0 = below_bf16(x0), r1 = below_bf16(x1);
-        b[i] = (int)hi16x2(r0, r1);
-        c[i] = (int)hi16x2(below_bf16(r0), below_bf16(r1));
+        const uint32_t p = pack_bf16x2(x0, x1);
+        const float r0 = x0 - bitsf(p << 16), r1 = x1 - bitsf(p & 0xffff0000u);
+        const uint32_t q = pack_bf16x2(r0, r1);
+        a[i] = (int)p;
+        b[i] = (int)q;
+        c[i] = (int)hi16x2(r0 - bitsf(q << 16), r1 - bitsf(q & 0xffff0000u));  // exact: at most 8 bits are left
     }
 }
 // Softmax in base 2: a weight is exp2(fma(score, c, -m)) with
