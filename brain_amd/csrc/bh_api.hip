@@ -13,6 +13,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <functional>
+#include <list>
 #include <map>
 #include <tuple>
 #include <mutex>
@@ -23,6 +24,7 @@
 #include "../../include/brain_hip.h"
 #include "bh_common.h"
 #include "bh_kv8.h"
+#include "bh_ws.h"
 
 namespace bh {
 hipError_t launch_max_abs_rows(hipStream_t s, const float* x, int m, int k, float* sx);
@@ -63,33 +65,47 @@ hipError_t launch_gemv_q4(hipStream_t s, const uint32_t* xq, const uint32_t* wq,
 hipError_t launch_gemm_q4(hipStream_t s, const uint32_t* xq, const uint32_t* wq, const float* sx,
                           const float* sw, const float* bias, void* out, int out_dtype, int m, int k, int n);
 
-// Split-K workspace, one per (device, stream): the S partial slabs of a
-// split GEMM. Every split kernel overwrites the slabs it uses before the
-// reduction reads them, so the buffer is never cleared. Calls on one stream
-// are ordered, so they never share it concurrently; a graph captured on the
-// stream replays in that stream's order too.
-struct SplitWs {
+// Workspaces, per (device, stream): what one kernel of a call leaves for the
+// next (the slabs of a split GEMM, padded operands, packed rows). Every call
+// writes what it reads, so they are never cleared. Calls on one stream run in
+// order; a call holds the stream's lock (WsLock) from its first launch on a
+// workspace to its last, so that the launches of two host threads on one
+// stream do not mix.
+struct StreamWs {
     int device;
     hipStream_t stream;
-    int slot;  // 0: split-K slabs, 1: W4A8 weights expanded to int8
-    int* ws;
-    size_t ints;
+    std::recursive_mutex launch;
+    struct {
+        int* ws;
+        size_t ints;
+    } slot[WS_SLOTS];
+    StreamWs(int d, hipStream_t s) : device(d), stream(s), slot{} {}
 };
-static std::mutex g_ws_mu;
-static std::vector<SplitWs> g_ws;
+static std::mutex g_ws_mu;  // guards the list; its elements stay where they are
+static std::list<StreamWs> g_ws;
 
-int* splitk_workspace(hipStream_t st, size_t ints, hipError_t* err, int slot) {
+static StreamWs* stream_ws(hipStream_t st, hipError_t* err) {
     int dev = 0;
     *err = hipGetDevice(&dev);
     if (*err != hipSuccess) return nullptr;
     std::lock_guard<std::mutex> g(g_ws_mu);
-    SplitWs* w = nullptr;
     for (auto& x : g_ws)
-        if (x.device == dev && x.stream == st && x.slot == slot) w = &x;
-    if (!w) {
-        g_ws.push_back(SplitWs{dev, st, slot, nullptr, 0});
-        w = &g_ws.back();
-    }
+        if (x.device == dev && x.stream == st) return &x;
+    g_ws.emplace_back(dev, st);
+    return &g_ws.back();
+}
+
+hipError_t WsLock::take(hipStream_t s) {
+    hipError_t err = hipSuccess;
+    if (StreamWs* w = stream_ws(s, &err)) lock_ = std::unique_lock<std::recursive_mutex>(w->launch);
+    return err;
+}
+
+int* splitk_workspace(hipStream_t st, size_t ints, hipError_t* err, int slot) {
+    StreamWs* sw = stream_ws(st, err);
+    if (!sw) return nullptr;
+    std::lock_guard<std::recursive_mutex> g(sw->launch);
+    auto* w = &sw->slot[slot];
     if (w->ints < ints) {
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone) {

@@ -29,6 +29,7 @@
 #include <type_traits>
 
 #include "bh_common.h"
+#include "bh_ws.h"
 
 namespace bh {
 
@@ -1202,10 +1203,6 @@ static inline bool gemm_aligned(const void* xq, const void* wq, int kg) {
            ((reinterpret_cast<uintptr_t>(wq) & 15u) == 0);
 }
 
-// Split-K workspace of the stream: at least `ints` i32 (grown outside graph
-// capture only; hipErrorStreamCaptureUnsupported otherwise).
-int* splitk_workspace(hipStream_t s, size_t ints, hipError_t* err, int slot = 0);
-
 // Workspace elements the GEMM needs for this shape (0 = no split-K).
 static int column_split(int m, int kg, int n, const TileChoice& tc, bool dma);
 
@@ -1255,6 +1252,8 @@ static hipError_t run_gemm(hipStream_t s, bool al, bool dma, const TileChoice& t
                            int* ws_fixed = nullptr) {
     if (tc.splits <= 1) return go_cfg<OUT, HAS_BIAS, STATIC>(s, al, dma, tc, a);
     hipError_t err = hipSuccess;
+    WsLock lock;  // over the split kernel and the reduction
+    if (!ws_fixed && (err = lock.take(s)) != hipSuccess) return err;
     a.ws = ws_fixed ? ws_fixed : splitk_workspace(s, (size_t)tc.splits * a.m * a.n, &err);
     if (!a.ws) return err == hipSuccess ? hipErrorOutOfMemory : err;
     a.splits = tc.splits;
@@ -1343,13 +1342,15 @@ __global__ __launch_bounds__(256) void pad_rows_kernel(const uint32_t* x, const 
 }
 
 // Pads both operands into the stream's workspace; false if that is not to be
-// had (the caller then takes the register-staged kernel), or *err set.
-static bool pad_operands(hipStream_t s, const uint32_t** xq, const uint32_t** wq, int m, int n, PadShape px, PadShape pw,
-                         hipError_t* err) {
+// had (the caller then takes the register-staged kernel), or *err set. The
+// caller keeps `lock` until the GEMM that reads them is launched.
+static bool pad_operands(hipStream_t s, WsLock& lock, const uint32_t** xq, const uint32_t** wq, int m, int n,
+                         PadShape px, PadShape pw, hipError_t* err) {
     *err = hipSuccess;
     const size_t ints = (size_t)m * px.kp + (size_t)n * pw.kp;
     if (ints * 4 > PAD_MAX_BYTES) return false;
-    int* ws = splitk_workspace(s, ints, err, 1);
+    if ((*err = lock.take(s)) != hipSuccess) return false;
+    int* ws = splitk_workspace(s, ints, err, WS_PAD);
     if (!ws) {
         if (*err == hipErrorStreamCaptureUnsupported) {
             (void)hipGetLastError();
@@ -1378,10 +1379,11 @@ size_t gemm_pad_workspace_ints(int m, int kg, int n) {
 
 hipError_t launch_gemm_i8(hipStream_t s, const uint32_t* xq, const uint32_t* wq, const float* sx,
                           const float* sw, const float* bias, void* out, int out_dtype, int m, int kg, int n) {
+    WsLock lock;
     if (kg > 0 && !(gemm_aligned(xq, wq, kg) && (kg * 4) % 128 == 0)) {
         const PadShape p = pad_shape(kg, 32);
         hipError_t err;
-        if (pad_operands(s, &xq, &wq, m, n, p, p, &err)) kg = p.kp;
+        if (pad_operands(s, lock, &xq, &wq, m, n, p, p, &err)) kg = p.kp;
         else if (err != hipSuccess) return err;
     }
     GemmArgs a{xq, wq, sx, sw, bias, out, m, kg, n, 0.f, 0.f, 1, nullptr};
@@ -1555,6 +1557,8 @@ static hipError_t run_q4(hipStream_t s, GemmArgs a) {
     const TileChoice tc = choose_tiles(a.m, a.kg, a.n);
     if (tc.splits > 1) {
         hipError_t err = hipSuccess;
+        WsLock lock;
+        if ((err = lock.take(s)) != hipSuccess) return err;
         a.ws = splitk_workspace(s, (size_t)tc.splits * a.m * a.n, &err);
         if (a.ws) {
             a.splits = tc.splits;
@@ -1573,12 +1577,13 @@ hipError_t launch_gemm_q4(hipStream_t s, const uint32_t* xq, const uint32_t* wq,
     // Aligned 16-byte loads need 16-byte rows in both operands: K % 32 == 0.
     const bool al = (k % 32) == 0 && ((reinterpret_cast<uintptr_t>(xq) | reinterpret_cast<uintptr_t>(wq)) & 15u) == 0;
     GemmArgs a{xq, wq, sx, sw, bias, out, m, k / 4, n, 0.f, 0.f, 1, nullptr};
+    WsLock lock;
     if (k > 0 && k + 127 < Q4_MAX_K) {
         bool ready = al && k % 128 == 0;
         if (!ready) {
             const PadShape px = pad_shape(k / 4, 32);
             hipError_t err;
-            ready = pad_operands(s, &a.xq, &a.wq, m, n, px, PadShape{k / 8, px.kp / 2}, &err);
+            ready = pad_operands(s, lock, &a.xq, &a.wq, m, n, px, PadShape{k / 8, px.kp / 2}, &err);
             if (ready) a.kg = px.kp;
             else if (err != hipSuccess) return err;
         }
@@ -1715,6 +1720,8 @@ hipError_t launch_gemm_i8_quant(hipStream_t s, const uint32_t* xq, const uint32_
     if (S >= 2 && S <= 4) {
         hipError_t err = hipSuccess;
         GemmArgs a{xq, wq, sx, sw, bias, out, m, kg, n, 0.f, 0.f, S, nullptr};
+        WsLock lock;
+        if ((err = lock.take(s)) != hipSuccess) return err;
         a.ws = splitk_workspace(s, (size_t)S * m * n, &err);
         if (a.ws) {
             err = go_dma<256, 256, 2, 4, 4, 64, OUT_I32, false, false, true, false, true>(s, a);
@@ -1827,7 +1834,9 @@ hipError_t launch_gemm_i8_gated(hipStream_t s, const uint32_t* xq, const uint32_
         const size_t pad = ((size_t)m + 63) / 64 * 64;
         const size_t ints = (size_t)m * kg + 3 * pad + pad / MOE_PACK_ROWS + 64;
         hipError_t err = hipSuccess;
-        int* ws = splitk_workspace(s, ints, &err, 3);
+        WsLock lock;
+        if ((err = lock.take(s)) != hipSuccess) return err;
+        int* ws = splitk_workspace(s, ints, &err, WS_MOE);
         if (ws) {
             uint32_t* cxq = reinterpret_cast<uint32_t*>(ws);
             float* csx = reinterpret_cast<float*>(ws + (size_t)m * kg);

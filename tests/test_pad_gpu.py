@@ -1,7 +1,11 @@
 """GEMMs whose rows the DMA kernel cannot read as they are (K % 128 != 0, or
 operands off by a word) run on zero-padded copies: accumulators against exact
 int64 sums around the 128-byte stage, for int8 and int4 weights; and a capture
-without a workspace, which takes the other kernel, against the eager bits."""
+without a workspace, which takes the other kernel, against the eager bits. The
+copies live in a workspace of the stream: two host threads on one stream do not
+mix theirs."""
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -69,3 +73,34 @@ def test_ragged_capture(gpu, q4, reserve):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, eager)
+
+
+def ragged(m, k, n, q4, seed):
+    rng = np.random.default_rng(seed)
+    x, w = words(rng, m, k // 4), words(rng, n, k // (8 if q4 else 4))
+    one = torch.ones(max(m, n), device="cuda")
+    want = torch.from_numpy((int8_of(x) @ (int4_of(w) if q4 else int8_of(w)).T).astype(np.int32)).cuda()
+    mm = ops.matmul_q4 if q4 else ops.matmul_i8
+    return (lambda: mm(x, w, one[:m], one[:n], None, torch.int32, "dyn")), want
+
+
+@pytest.mark.parametrize("m,k,n", [(65, 1000, 257), (40, 6152, 64)])  # unsplit; split over K
+def test_two_threads_on_one_stream(gpu, m, k, n):
+    work = [ragged(m, k, n, q4, seed) for seed, q4 in enumerate((False, True, False, True))]
+    torch.cuda.synchronize()
+    stream = torch.cuda.current_stream()
+    start, bad = threading.Barrier(len(work)), []
+
+    def run(call, want):
+        with torch.cuda.stream(stream):
+            start.wait()
+            outs = [call() for _ in range(50)]
+            torch.cuda.synchronize()
+            bad.extend(i for i, out in enumerate(outs) if not torch.equal(out, want))
+
+    threads = [threading.Thread(target=run, args=w) for w in work]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
