@@ -70,7 +70,8 @@ hipError_t launch_gemm_q4(hipStream_t s, const uint32_t* xq, const uint32_t* wq,
 // writes what it reads, so they are never cleared. Calls on one stream run in
 // order; a call holds the stream's lock (WsLock) from its first launch on a
 // workspace to its last, so that the launches of two host threads on one
-// stream do not mix.
+// stream do not mix. A captured launch keeps the capture stream's slabs or
+// packed rows; its graph is ordered by the stream it is launched on.
 struct StreamWs {
     int device;
     hipStream_t stream;
@@ -383,22 +384,15 @@ int bh_matmul_i8_dyn_noalloc(void* stream, const uint32_t* xq, const uint32_t* w
 int bh_reserve_workspace(void* stream, uint32_t m, uint32_t kg, uint32_t n) {
     if ((uint64_t)kg * 4 > I32MAX || m > I32MAX || n > I32MAX)
         return fail(BH_ERR_INVALID, "bh_reserve_workspace: m=%u kg=%u n=%u out of range", m, kg, n);
-    // Both workspaces a GEMM of this shape may take: the split-K slabs
-    // (bh_matmul_i8_dyn, bh_matmul_i8_dyn_quant, W4A8) and, for K % 128 != 0,
-    // the zero-padded operands (whose GEMM is the padded shape's).
-    const size_t pad = gemm_pad_workspace_ints((int)m, (int)kg, (int)n);
-    size_t split = std::max(gemm_workspace_ints((int)m, (int)kg, (int)n), gemm_quant_workspace_ints((int)m, (int)kg, (int)n));
-    if (pad) split = std::max(split, gemm_workspace_ints((int)m, ((int)kg + 31) / 32 * 32, (int)n));
-    const size_t need[2] = {split, pad};
-    for (int slot = 0; slot < 2; ++slot) {
-        if (!need[slot]) continue;
-        hipError_t err = hipSuccess;
-        if (!splitk_workspace((hipStream_t)stream, need[slot], &err, slot)) {
-            if (err == hipErrorStreamCaptureUnsupported)
-                return fail(BH_ERR_INVALID, "bh_reserve_workspace: stream is capturing; reserve before capture");
-            return fail(err == hipErrorOutOfMemory ? BH_ERR_NOMEM : BH_ERR_HIP, "bh_reserve_workspace: %s",
-                        hipGetErrorString(err));
-        }
+    // The split-K slabs (bh_matmul_i8_dyn, bh_matmul_i8_dyn_quant, W4A8) of the
+    // shape as it is captured: unpadded.
+    const size_t need = std::max(gemm_workspace_ints((int)m, (int)kg, (int)n), gemm_quant_workspace_ints((int)m, (int)kg, (int)n));
+    hipError_t err = hipSuccess;
+    if (need && !splitk_workspace((hipStream_t)stream, need, &err)) {
+        if (err == hipErrorStreamCaptureUnsupported)
+            return fail(BH_ERR_INVALID, "bh_reserve_workspace: stream is capturing; reserve before capture");
+        return fail(err == hipErrorOutOfMemory ? BH_ERR_NOMEM : BH_ERR_HIP, "bh_reserve_workspace: %s",
+                    hipGetErrorString(err));
     }
     return BH_OK;
 }

@@ -1309,10 +1309,23 @@ static int column_split(int m, int kg, int n, const TileChoice& tc, bool dma) {
 // staged -> copy + DMA kernel): 40x60x130 10.0 -> 2.6 + 3.4 us, 64x520x1024
 // 24.4 -> 2.9 + 5.2, 2000x132x4000 21.7 -> 3.4 + 11.1, 333x2900x1111 51.6 ->
 // 6.2 + 11.2; 2000x5000x5000 220 -> 90 us for the whole linear.
-// The workspace for it is bounded; larger operands, a stream under capture
-// whose workspace is too small and the no-allocation entry take the
-// register-staged kernel.
+// The workspace for it is bounded; larger operands, a stream under capture and
+// the no-allocation entry take the register-staged kernel.
 constexpr size_t PAD_MAX_BYTES = size_t(512) << 20;
+
+// Whether a call that can do without may use the stream's workspace. Not under
+// capture: the graph's launches are ordered by the stream it is launched on,
+// not by the one it was captured on, so two graphs, or a graph and eager
+// calls, would share the buffer unordered. Not on the per-thread default
+// stream: its handle is one stream per thread, so the buffer would be shared
+// by unordered streams as well.
+static bool workspace_optional(hipStream_t s) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (s == hipStreamPerThread) return false;
+    if (hipStreamIsCapturing(s, &cs) == hipSuccess) return cs == hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return false;
+}
 
 struct PadShape {
     int kg, kp;  // words of a row, and of a padded row (a multiple of 4)
@@ -1348,16 +1361,11 @@ static bool pad_operands(hipStream_t s, WsLock& lock, const uint32_t** xq, const
                          PadShape px, PadShape pw, hipError_t* err) {
     *err = hipSuccess;
     const size_t ints = (size_t)m * px.kp + (size_t)n * pw.kp;
-    if (ints * 4 > PAD_MAX_BYTES) return false;
+    if (ints * 4 > PAD_MAX_BYTES || !workspace_optional(s)) return false;
     if ((*err = lock.take(s)) != hipSuccess) return false;
     int* ws = splitk_workspace(s, ints, err, WS_PAD);
     if (!ws) {
-        if (*err == hipErrorStreamCaptureUnsupported) {
-            (void)hipGetLastError();
-            *err = hipSuccess;
-        } else if (*err == hipSuccess) {
-            *err = hipErrorOutOfMemory;
-        }
+        if (*err == hipSuccess) *err = hipErrorOutOfMemory;
         return false;
     }
     const int64_t cx = (int64_t)m * (px.kp / 4), ct = (int64_t)(ints / 4);
@@ -1367,14 +1375,6 @@ static bool pad_operands(hipStream_t s, WsLock& lock, const uint32_t** xq, const
     *xq = reinterpret_cast<const uint32_t*>(ws);
     *wq = *xq + (size_t)m * px.kp;
     return true;
-}
-
-// Workspace elements (slot 1) of the padded operands of a shape: int8 rows
-// (W8A8), or int8 and int4 rows (W4A8); 0 where they are not padded.
-size_t gemm_pad_workspace_ints(int m, int kg, int n) {
-    const PadShape p = pad_shape(kg, 32);
-    const size_t ints = ((size_t)m + n) * p.kp;  // covers W4A8, whose weight rows are half as long
-    return p.kp != kg && ints * 4 <= PAD_MAX_BYTES ? ints : 0;
 }
 
 hipError_t launch_gemm_i8(hipStream_t s, const uint32_t* xq, const uint32_t* wq, const float* sx,
@@ -1531,9 +1531,29 @@ hipError_t launch_gemm_i8_static(hipStream_t s, const uint32_t* xq, const uint32
 // 64x4096x4096 42 -> 23 us, 128x4096x11008 45 -> 34.
 // Anything else: the register-staged kernel with int4 B unpacked on the way
 // into LDS.
+//
+// From this many rows a W4A8 GEMM may split K into the stream's slabs under
+// capture too, where the caller has reserved them; fewer rows are one launch
+// without shared memory there (workspace_optional).
+constexpr int Q4_CAPTURE_SPLIT_M = 256;
+
+static bool q4_may_split(hipStream_t s, int m) { return m >= Q4_CAPTURE_SPLIT_M || workspace_optional(s); }
+
 template <int OUT, bool HAS_BIAS>
-static hipError_t go_q4(hipStream_t s, bool aligned, const GemmArgs& a) {
-    TileChoice tc = choose_tiles(a.m, a.kg, a.n);
+static hipError_t go_q4(hipStream_t s, bool aligned, GemmArgs a) {
+    const TileChoice tc = choose_tiles(a.m, a.kg, a.n);
+    if (aligned && a.m >= Q4_CAPTURE_SPLIT_M && tc.splits > 1) {
+        hipError_t err = hipSuccess;
+        WsLock lock;
+        if ((err = lock.take(s)) != hipSuccess) return err;
+        a.ws = splitk_workspace(s, (size_t)tc.splits * a.m * a.n, &err);
+        if (a.ws) {
+            a.splits = tc.splits;
+            if ((err = go<128, 128, 2, 2, OUT_I32, false, false, true, true>(s, aligned, a)) != hipSuccess) return err;
+            return reduce_splits<OUT, HAS_BIAS, false>(s, a);
+        }
+        (void)hipGetLastError();  // without the slabs: unsplit
+    }
     if (tc.cfg == TILE_256) return go<256, 256, 2, 2, OUT, HAS_BIAS, false, false, true>(s, aligned, a);
     return go<128, 128, 2, 2, OUT, HAS_BIAS, false, false, true>(s, aligned, a);
 }
@@ -1555,7 +1575,7 @@ static hipError_t go_q4_dma(hipStream_t s, int cfg, const GemmArgs& a) {
 template <int OUT, bool HAS_BIAS>
 static hipError_t run_q4(hipStream_t s, GemmArgs a) {
     const TileChoice tc = choose_tiles(a.m, a.kg, a.n);
-    if (tc.splits > 1) {
+    if (tc.splits > 1 && q4_may_split(s, a.m)) {
         hipError_t err = hipSuccess;
         WsLock lock;
         if ((err = lock.take(s)) != hipSuccess) return err;

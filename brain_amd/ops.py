@@ -200,9 +200,10 @@ def f32_to_bf16(x):
 
 
 def reserve_workspace(m, k, n, stream=None):
-    """Pre-size the workspaces of `stream` (default: current) that an
-    [m,k] x [n,k] GEMM may take (split-K slabs; for k % 128 != 0 the
-    zero-padded operands); required before capturing a GEMM that splits K."""
+    """Pre-size the split-K slabs of `stream` (default: current) that an
+    [m,k] x [n,k] GEMM may take; required before capturing a GEMM that splits K
+    in a graph, which must then not run concurrently with other work that uses
+    the stream's slabs."""
     sp = (stream or torch.cuda.current_stream()).cuda_stream
     check(load().bh_reserve_workspace(sp, m, k // 4, n))
 

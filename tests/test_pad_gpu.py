@@ -1,9 +1,9 @@
 """GEMMs whose rows the DMA kernel cannot read as they are (K % 128 != 0, or
 operands off by a word) run on zero-padded copies: accumulators against exact
-int64 sums around the 128-byte stage, for int8 and int4 weights; and a capture
-without a workspace, which takes the other kernel, against the eager bits. The
-copies live in a workspace of the stream: two host threads on one stream do not
-mix theirs."""
+int64 sums around the 128-byte stage, for int8 and int4 weights. The copies live
+in a workspace of the stream: two host threads on one stream do not mix theirs,
+and a captured GEMM does not use it (it takes the other kernel): against the
+eager bits, with graphs replayed on several streams at once."""
 import threading
 
 import numpy as np
@@ -104,3 +104,70 @@ def test_two_threads_on_one_stream(gpu, m, k, n):
     for t in threads:
         t.join()
     assert not bad
+
+
+def test_two_graphs_of_one_capture_stream(gpu):
+    m, k, n = 65, 1000, 257
+    cap = torch.cuda.Stream()
+    work = [ragged(m, k, n, q4, 11 + q4) for q4 in (False, True)] + [ragged(m, k, n, False, 13)]
+    torch.cuda.synchronize()
+    graphs = []
+    with torch.cuda.stream(cap):
+        for call, want in work:
+            assert torch.equal(call(), want)  # the stream's workspace is large enough
+    for call, _ in work[:2]:
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=cap):
+            graphs.append((g, call()))
+    s0, s1 = torch.cuda.Stream(), torch.cuda.Stream()
+    for _ in range(20):
+        for _, out in graphs:
+            out.fill_(0)
+        torch.cuda.synchronize()
+        for s, (g, _) in zip((s0, s1), graphs):
+            with torch.cuda.stream(s):
+                g.replay()
+        with torch.cuda.stream(cap):  # eager work that does use the workspace
+            assert torch.equal(work[2][0](), work[2][1])
+        torch.cuda.synchronize()
+        for (_, out), (_, want) in zip(graphs, work):
+            assert torch.equal(out, want)
+
+
+def test_capture_after_a_larger_ragged_call(gpu):
+    """33x2692x1024 does not split K, its padded K = 2816 does: captured without
+    a reserve after an eager call that left a larger padded copy, it runs."""
+    cap = torch.cuda.Stream()
+    call, want = ragged(33, 2692, 1024, False, 3)
+    large, _ = ragged(1056, 2692, 1024, False, 4)  # padded, unsplit: no slabs are left behind
+    torch.cuda.synchronize()
+    with torch.cuda.stream(cap):
+        large()
+    cap.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=cap):
+        out = call()
+    for _ in range(3):
+        out.fill_(0)
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+
+
+def test_captured_q4_splits_from_256_rows_only(gpu):
+    """int4 weights under capture with the slabs reserved: from 256 rows K is
+    split (K % 128 == 0 on the DMA tiles, else on the register-staged ones),
+    below it is not. Exact sums either way."""
+    for m, k, n in ((256, 8160, 1024), (256, 8192, 1024), (200, 8192, 1024)):
+        cap = torch.cuda.Stream()
+        call, want = ragged(m, k, n, True, m + k)
+        ops.reserve_workspace(m, k, n, cap)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=cap):
+            out = call()
+        for _ in range(3):
+            out.fill_(0)
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want), (m, k, n)

@@ -187,6 +187,23 @@ def test_chunking_and_graph_are_bit_identical(gpu):
     b.close()
 
 
+def test_captured_decode_with_a_ragged_down_projection(gpu):
+    """d_ff = 2692, 33 rows: the down projection does not split K as it is and
+    would after padding to 2816. The prompt (1056 rows) runs it padded and
+    unsplit; the captured decode must run all the same, to the eager bits."""
+    cfg = dict(SMALL, vocab=256, n_layers=1, d_model=1024, d_ff=2692)
+    w = scaled_weights(cfg, 17)
+    prompts = np.random.default_rng(17).integers(0, 256, (33, 32)).astype(np.uint32)
+    got = []
+    for eager in (False, True):
+        e = engine_for(cfg, w, 33, 40)
+        e.prefill(prompts)
+        got.append((e.decode(3, eager=eager), e.logits()))
+        e.close()
+    assert (got[0][0] == got[1][0]).all()
+    assert (got[0][1].view(np.uint32) == got[1][1].view(np.uint32)).all()
+
+
 def test_engine_argument_errors(gpu):
     from brain_amd._lib import BrainHipError
     e = Qwen3Engine(SMALL, 2, 16)
