@@ -76,12 +76,11 @@ struct StreamWs {
     int device;
     hipStream_t stream;
     std::recursive_mutex launch;
-    struct {
-        int* ws;
-        size_t ints;
-    } slot[WS_SLOTS];
-    StreamWs(int d, hipStream_t s) : device(d), stream(s), slot{} {}
+    WsBuf slot[WS_SLOTS];
+    StreamWs(int d, hipStream_t s) : device(d), stream(s) {}
 };
+// What a workspace may double to; a single call's need may be larger.
+static const size_t WS_CAP_BYTES[WS_SLOTS] = {SPLITK_MAX_BYTES, PAD_MAX_BYTES, SIZE_MAX};
 static std::mutex g_ws_mu;  // guards the list; its elements stay where they are
 static std::list<StreamWs> g_ws;
 
@@ -106,23 +105,28 @@ int* splitk_workspace(hipStream_t st, size_t ints, hipError_t* err, int slot) {
     StreamWs* sw = stream_ws(st, err);
     if (!sw) return nullptr;
     std::lock_guard<std::recursive_mutex> g(sw->launch);
-    auto* w = &sw->slot[slot];
-    if (w->ints < ints) {
+    WsBuf& w = sw->slot[slot];
+    if (w.ints < ints) {
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone) {
             // No allocation inside a capture: the caller reserves beforehand.
             *err = hipErrorStreamCaptureUnsupported;
             return nullptr;
         }
-        // Growing. The old buffer is kept, not freed, until the process ends:
-        // a HIP graph captured earlier may still launch kernels that use it.
-        // (Sizes only grow and each is capped, so this retains little.)
-        int* nb = nullptr;
-        if ((*err = hipMalloc(&nb, ints * 4)) != hipSuccess) return nullptr;
-        w->ws = nb;
-        w->ints = ints;
+        // A capture of another stream is none of this allocation's business
+        // (without the exchange it would fail, and end that capture).
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        if ((*err = hipThreadExchangeStreamCaptureMode(&mode)) != hipSuccess) return nullptr;
+        const bool ok = ws_grow(w, ints, WS_CAP_BYTES[slot] / 4, [&](size_t bytes) {
+            void* p = nullptr;
+            *err = hipMalloc(&p, bytes);
+            if (*err != hipSuccess) (void)hipGetLastError();
+            return *err == hipSuccess ? p : nullptr;
+        });
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        if (!ok) return nullptr;
     }
-    return w->ws;
+    return w.ws;
 }
 
 // ---------------------------------------------------------------- small kernels

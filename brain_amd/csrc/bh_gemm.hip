@@ -1008,8 +1008,6 @@ static int t32x64_env() {
 // Sums of int8 x 16 q stay inside i32 below this K: K * 128 * 8 * 16 < 2^31.
 constexpr int Q4_MAX_K = 131072;
 
-constexpr size_t SPLITK_MAX_BYTES = size_t(64) << 20;  // workspace cap per call
-
 // Split-K. Measured on MI355X, a tile alone on its CU costs a few us fixed
 // (launch, first loads, epilogue) plus P us per 64-byte K stage (0.25 for
 // 128x128, 0.18 for the 64-row tiles), so splitting K S ways shortens the
@@ -1311,7 +1309,6 @@ static int column_split(int m, int kg, int n, const TileChoice& tc, bool dma) {
 // 6.2 + 11.2; 2000x5000x5000 220 -> 90 us for the whole linear.
 // The workspace for it is bounded; larger operands, a stream under capture and
 // the no-allocation entry take the register-staged kernel.
-constexpr size_t PAD_MAX_BYTES = size_t(512) << 20;
 
 // Whether a call that can do without may use the stream's workspace. Not under
 // capture: the graph's launches are ordered by the stream it is launched on,
