@@ -1253,7 +1253,11 @@ static hipError_t run_gemm(hipStream_t s, bool al, bool dma, const TileChoice& t
     WsLock lock;  // over the split kernel and the reduction
     if (!ws_fixed && (err = lock.take(s)) != hipSuccess) return err;
     a.ws = ws_fixed ? ws_fixed : splitk_workspace(s, (size_t)tc.splits * a.m * a.n, &err);
-    if (!a.ws) return err == hipSuccess ? hipErrorOutOfMemory : err;
+    if (!a.ws) {
+        // No memory for the slabs: the same tiles, unsplit.
+        if (err == hipErrorOutOfMemory) return go_cfg<OUT, HAS_BIAS, STATIC>(s, al, dma, tc, a);
+        return err;
+    }
     a.splits = tc.splits;
     if (dma && tc.cfg == TILE_256)
         err = go_dma<256, 256, 2, 4, 4, 64, OUT_I32, false, false, true, false, true>(s, a);
@@ -1361,8 +1365,8 @@ static bool pad_operands(hipStream_t s, WsLock& lock, const uint32_t** xq, const
     if (ints * 4 > PAD_MAX_BYTES || !workspace_optional(s)) return false;
     if ((*err = lock.take(s)) != hipSuccess) return false;
     int* ws = splitk_workspace(s, ints, err, WS_PAD);
-    if (!ws) {
-        if (*err == hipSuccess) *err = hipErrorOutOfMemory;
+    if (!ws) {  // no memory: the other kernel needs none
+        *err = hipSuccess;
         return false;
     }
     const int64_t cx = (int64_t)m * (px.kp / 4), ct = (int64_t)(ints / 4);
@@ -1582,8 +1586,8 @@ static hipError_t run_q4(hipStream_t s, GemmArgs a) {
             if ((err = go_q4_dma<OUT_I32, false, true>(s, tc.cfg, a)) != hipSuccess) return err;
             return reduce_splits<OUT, HAS_BIAS, false>(s, a);
         }
-        // Capturing without the workspace: the same tiles, unsplit.
-        if (err != hipErrorStreamCaptureUnsupported) return err == hipSuccess ? hipErrorOutOfMemory : err;
+        // Capturing without the slabs, or no memory for them: the same tiles, unsplit.
+        if (err != hipErrorStreamCaptureUnsupported && err != hipErrorOutOfMemory) return err;
         (void)hipGetLastError();
     }
     return go_q4_dma<OUT, HAS_BIAS, false>(s, tc.cfg, a);
@@ -1753,8 +1757,8 @@ hipError_t launch_gemm_i8_quant(hipStream_t s, const uint32_t* xq, const uint32_
             }
             return hipGetLastError();
         }
-        if (err != hipErrorStreamCaptureUnsupported) return err == hipSuccess ? hipErrorOutOfMemory : err;
-        (void)hipGetLastError();  // capturing without the workspace: the unfused pair below
+        if (err != hipErrorStreamCaptureUnsupported && err != hipErrorOutOfMemory) return err;
+        (void)hipGetLastError();  // without the workspace: the unfused pair below
     }
     hipError_t err = launch_gemm_i8(s, xq, wq, sx, sw, bias, out, OUT_BF16, m, kg, n);
     if (err != hipSuccess) return err;
