@@ -50,6 +50,7 @@ hipError_t launch_gemm_i8_noalloc(hipStream_t s, const uint32_t* xq, const uint3
                                   const float* sw, const float* bias, void* out, int out_dtype, int m, int kg, int n,
                                   size_t* need_bytes);
 size_t noalloc_scratch_bytes();
+size_t gemm_q4_expand_ints(int m, int k, int n);
 size_t gemm_pad_workspace_ints(int m, int kg, int n);
 hipError_t launch_gemv_i8_gated(hipStream_t s, const uint32_t* xq, const uint32_t* wq, const float* sx,
                                 const float* sw, const float* gate, int gate_stride, int gate_col, float* out, int m,
@@ -80,7 +81,7 @@ struct StreamWs {
     StreamWs(int d, hipStream_t s) : device(d), stream(s) {}
 };
 // What a workspace may double to; a single call's need may be larger.
-static const size_t WS_CAP_BYTES[WS_SLOTS] = {SPLITK_MAX_BYTES, PAD_MAX_BYTES, SIZE_MAX};
+static const size_t WS_CAP_BYTES[WS_SLOTS] = {SPLITK_MAX_BYTES, PAD_MAX_BYTES, SIZE_MAX, PAD_MAX_BYTES};
 static std::mutex g_ws_mu;  // guards the list; its elements stay where they are
 static std::list<StreamWs> g_ws;
 
@@ -398,6 +399,9 @@ int bh_reserve_workspace(void* stream, uint32_t m, uint32_t kg, uint32_t n) {
         return fail(err == hipErrorOutOfMemory ? BH_ERR_NOMEM : BH_ERR_HIP, "bh_reserve_workspace: %s",
                     hipGetErrorString(err));
     }
+    // The expanded weights of an int4 GEMM (which can do without).
+    if (const size_t w8 = gemm_q4_expand_ints((int)m, (int)kg * 4, (int)n))
+        (void)splitk_workspace((hipStream_t)stream, w8, &err, WS_EXPAND);
     return BH_OK;
 }
 

@@ -1526,9 +1526,9 @@ hipError_t launch_gemm_i8_static(hipStream_t s, const uint32_t* xq, const uint32
 // the tiles of the int8 GEMM in their 128-byte-stage forms. The unpacking (10
 // vector instructions per 32 x 16-byte fragment) runs beside the MFMAs it
 // feeds, and B moves half the bytes. Expanding the weights to int8 in memory
-// first (as from 256 rows before) cost 1.5 N K bytes of traffic on every call:
-// 512x4096x11008 13.6 + 34.9 us -> 39.0; the register-staged kernel, before
-// that the one below 256 rows, has one 128x128 tile shape: whole linears at
+// first costs 1.5 N K bytes of traffic on every call (512x4096x11008 13.6 +
+// 34.9 us -> 39.0 unpacking) and is kept for the most rows (Q4_EXPAND_M); the
+// register-staged kernel has 128x128 and 256x256 tiles only: whole linears at
 // 64x4096x4096 42 -> 23 us, 128x4096x11008 45 -> 34.
 // Anything else: the register-staged kernel with int4 B unpacked on the way
 // into LDS.
@@ -1573,9 +1573,14 @@ static hipError_t go_q4_dma(hipStream_t s, int cfg, const GemmArgs& a) {
     }
 }
 
+// hipErrorNotSupported: K is too long for one i32 sum of 16 q and there are no
+// slabs to split it over.
 template <int OUT, bool HAS_BIAS>
 static hipError_t run_q4(hipStream_t s, GemmArgs a) {
-    const TileChoice tc = choose_tiles(a.m, a.kg, a.n);
+    TileChoice tc = choose_tiles(a.m, a.kg, a.n);
+    const int smin = a.kg * 4 / (Q4_MAX_K - 1024) + 1;  // a split ends on a stage: up to 256 longer than K / S
+    tc.splits = std::max(tc.splits, smin);
+    if (smin > 1 && (double)tc.splits * a.m * a.n * 4 > (double)SPLITK_MAX_BYTES) return hipErrorNotSupported;
     if (tc.splits > 1 && q4_may_split(s, a.m)) {
         hipError_t err = hipSuccess;
         WsLock lock;
@@ -1590,30 +1595,111 @@ static hipError_t run_q4(hipStream_t s, GemmArgs a) {
         if (err != hipErrorStreamCaptureUnsupported && err != hipErrorOutOfMemory) return err;
         (void)hipGetLastError();
     }
+    if (smin > 1) return hipErrorNotSupported;
     return go_q4_dma<OUT, HAS_BIAS, false>(s, tc.cfg, a);
+}
+
+static hipError_t run_q4_out(hipStream_t s, int out_dtype, const GemmArgs& a) {
+    switch (out_dtype) {
+        case OUT_I32: return run_q4<OUT_I32, false>(s, a);
+        case OUT_F32: return a.bias ? run_q4<OUT_F32, true>(s, a) : run_q4<OUT_F32, false>(s, a);
+        default: return a.bias ? run_q4<OUT_BF16, true>(s, a) : run_q4<OUT_BF16, false>(s, a);
+    }
+}
+
+// Columns [n0, n0 + nn) of a call; row_words: the words of a weight row.
+static GemmArgs q4_columns(const GemmArgs& a, int out_dtype, int row_words, int n0, int nn) {
+    GemmArgs t = a;
+    t.n = nn;
+    t.ldo = (int)out_ld(a);
+    t.wq = a.wq + (size_t)n0 * row_words;
+    t.sw = a.sw ? a.sw + n0 : nullptr;
+    t.bias = a.bias ? a.bias + n0 : nullptr;
+    t.out = static_cast<uint8_t*>(a.out) + (size_t)n0 * (out_dtype == OUT_BF16 ? 2 : 4);
+    return t;
+}
+
+// From this many rows the int4 weights are expanded to int8 in memory first
+// (1.5 N K bytes of traffic, the same for any row count) and the int8 GEMM runs
+// on them, which multiplies a little faster than the tiles that unpack
+// (M x K x N, whole linear, unpacking -> expanded: 8192x4096x11008 432 -> 426
+// us, 6144x4096x11008 369.5 -> 364, 6144x4096x4096 149.6 -> 147.2;
+// 4096x4096x4096, product alone, 75.6 -> 80.2, 4096x4096x11008 199 -> 203,
+// 2048x4096x11008 133 -> 140).
+constexpr int Q4_EXPAND_M = 6144;
+
+__global__ __launch_bounds__(256) void expand_q4_kernel(const v4i* w4, v4i* w8, int64_t pieces) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < pieces; i += (int64_t)gridDim.x * 256) {
+        v4i lo, hi;
+        unpack_q4x4(w4[i], lo, hi);
+        w8[2 * i] = lo;
+        w8[2 * i + 1] = hi;
+    }
+}
+
+// Elements of the workspace (WS_EXPAND) for the expanded weights.
+size_t gemm_q4_expand_ints(int m, int k, int n) {
+    return m >= Q4_EXPAND_M && k % 128 == 0 ? (size_t)n * (k / 4) : 0;
+}
+
+// hipErrorNotSupported: no workspace for it (under capture it has to be
+// reserved; it is then the graph's, like slabs).
+static hipError_t launch_q4_expanded(hipStream_t s, int out_dtype, const GemmArgs& a) {
+    hipError_t err = hipSuccess;
+    WsLock lock;
+    if ((err = lock.take(s)) != hipSuccess) return err;
+    int* w8 = splitk_workspace(s, gemm_q4_expand_ints(a.m, a.kg * 4, a.n), &err, WS_EXPAND);
+    if (!w8) return err == hipErrorStreamCaptureUnsupported || err == hipErrorOutOfMemory ? hipErrorNotSupported : err;
+    const int64_t pieces = (int64_t)a.n * a.kg / 8;
+    const unsigned grid = (unsigned)std::min<int64_t>((pieces + 255) / 256, 256 * 8);
+    expand_q4_kernel<<<grid, 256, 0, s>>>(reinterpret_cast<const v4i*>(a.wq), reinterpret_cast<v4i*>(w8), pieces);
+    if ((err = hipGetLastError()) != hipSuccess) return err;
+    err = launch_gemm_i8(s, a.xq, reinterpret_cast<const uint32_t*>(w8), a.sx, a.sw, a.bias, a.out, out_dtype, a.m,
+                         a.kg, a.n);
+    return err == hipErrorStreamCaptureUnsupported ? hipErrorNotSupported : err;  // its slabs were not reserved
+}
+
+// Operands of whole 128-byte K stages, with the column split of the int8 GEMM
+// where its 256x256 tiles would leave most of a round empty (8192x4096x11008,
+// unpacking: 439 us as one grid, 417 split).
+static hipError_t launch_q4_dma(hipStream_t s, int out_dtype, const GemmArgs& a) {
+    const int n_main = column_split(a.m, a.kg, a.n, choose_tiles(a.m, a.kg, a.n), a.kg * 4 < Q4_MAX_K - 1024);
+    if (!n_main) return run_q4_out(s, out_dtype, a);
+    const hipError_t err = run_q4_out(s, out_dtype, q4_columns(a, out_dtype, a.kg / 2, 0, n_main));
+    return err != hipSuccess ? err : run_q4_out(s, out_dtype, q4_columns(a, out_dtype, a.kg / 2, n_main, a.n - n_main));
 }
 
 hipError_t launch_gemm_q4(hipStream_t s, const uint32_t* xq, const uint32_t* wq, const float* sx,
                           const float* sw, const float* bias, void* out, int out_dtype, int m, int k, int n) {
     // Aligned 16-byte loads need 16-byte rows in both operands: K % 32 == 0.
     const bool al = (k % 32) == 0 && ((reinterpret_cast<uintptr_t>(xq) | reinterpret_cast<uintptr_t>(wq)) & 15u) == 0;
-    GemmArgs a{xq, wq, sx, sw, bias, out, m, k / 4, n, 0.f, 0.f, 1, nullptr};
-    WsLock lock;
-    if (k > 0 && k + 127 < Q4_MAX_K) {
-        bool ready = al && k % 128 == 0;
-        if (!ready) {
-            const PadShape px = pad_shape(k / 4, 32);
-            hipError_t err;
-            ready = pad_operands(s, lock, &a.xq, &a.wq, m, n, px, PadShape{k / 8, px.kp / 2}, &err);
-            if (ready) a.kg = px.kp;
-            else if (err != hipSuccess) return err;
-        }
-        if (ready) switch (out_dtype) {
-            case OUT_I32: return run_q4<OUT_I32, false>(s, a);
-            case OUT_F32: return bias ? run_q4<OUT_F32, true>(s, a) : run_q4<OUT_F32, false>(s, a);
-            default: return bias ? run_q4<OUT_BF16, true>(s, a) : run_q4<OUT_BF16, false>(s, a);
+    const GemmArgs a{xq, wq, sx, sw, bias, out, m, k / 4, n, 0.f, 0.f, 1, nullptr};
+    hipError_t err = hipErrorNotSupported;
+    if (k > 0 && al && k % 128 == 0) {
+        if (gemm_q4_expand_ints(m, k, n)) err = launch_q4_expanded(s, out_dtype, a);
+        if (err == hipErrorNotSupported) err = launch_q4_dma(s, out_dtype, a);
+    } else if (k > 0) {
+        // Padded, in as many column ranges as it takes to stay within the
+        // workspace's bound; more than one only where the register-staged
+        // kernel has nothing but large tiles to offer.
+        WsLock lock;
+        const PadShape px = pad_shape(k / 4, 32), pw{k / 8, px.kp / 2};
+        const int64_t left = (int64_t)(PAD_MAX_BYTES / 4) - (int64_t)m * px.kp;
+        int step = n;
+        if ((int64_t)n * pw.kp > left && al && m >= Q4_CAPTURE_SPLIT_M)
+            step = left > 0 ? (int)(left / pw.kp / 256 * 256) : 0;
+        for (int n0 = 0; step > 0 && n0 < n; n0 += step) {
+            GemmArgs t = q4_columns(a, out_dtype, k / 8, n0, std::min(step, n - n0));
+            if (!pad_operands(s, lock, &t.xq, &t.wq, m, t.n, px, pw, &err)) {
+                if (err == hipSuccess) err = hipErrorNotSupported;
+                break;
+            }
+            t.kg = px.kp;
+            if ((err = launch_q4_dma(s, out_dtype, t)) != hipSuccess) break;
         }
     }
+    if (err != hipErrorNotSupported) return err;
+    (void)hipGetLastError();
     switch (out_dtype) {
         case OUT_I32: return go_q4<OUT_I32, false>(s, al, a);
         case OUT_F32: return bias ? go_q4<OUT_F32, true>(s, al, a) : go_q4<OUT_F32, false>(s, al, a);

@@ -9,7 +9,8 @@
 namespace bh {
 
 // What a workspace holds.
-enum WsSlot { WS_SPLIT = 0, WS_PAD = 1, WS_MOE = 2, WS_SLOTS = 3 };  // split-K slabs, padded operands, packed MoE rows
+// split-K slabs, padded operands, packed MoE rows, int4 weights as int8
+enum WsSlot { WS_SPLIT = 0, WS_PAD = 1, WS_MOE = 2, WS_EXPAND = 3, WS_SLOTS = 4 };
 
 constexpr size_t SPLITK_MAX_BYTES = size_t(64) << 20;  // slabs of one call
 constexpr size_t PAD_MAX_BYTES = size_t(512) << 20;    // padded operands of one call

@@ -200,10 +200,11 @@ def f32_to_bf16(x):
 
 
 def reserve_workspace(m, k, n, stream=None):
-    """Pre-size the split-K slabs of `stream` (default: current) that an
-    [m,k] x [n,k] GEMM may take; required before capturing a GEMM that splits K
+    """Pre-size the workspaces of `stream` (default: current) that an
+    [m,k] x [n,k] GEMM may take (split-K slabs; from 6144 rows the int8
+    expansion of int4 weights); required before capturing a GEMM that splits K
     in a graph, which must then not run concurrently with other work that uses
-    the stream's slabs."""
+    the stream's workspaces."""
     sp = (stream or torch.cuda.current_stream()).cuda_stream
     check(load().bh_reserve_workspace(sp, m, k // 4, n))
 

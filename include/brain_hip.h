@@ -136,15 +136,16 @@ int bh_matmul_i8_dyn_noalloc(void* stream, const uint32_t* xq, const uint32_t* w
                              const float* sw, const float* bias, void* out, int out_dtype, uint32_t m, uint32_t kg,
                              uint32_t n);
 
-/* Pre-size the library-held split-K workspace of `stream` for a
- * bh_matmul_i8_dyn or bh_matmul_q4_dyn call of this shape (a no-op for shapes
- * that do not split K). The workspace is allocated per (device, stream) on
+/* Pre-size the library-held workspaces of `stream` for a bh_matmul_i8_dyn or
+ * bh_matmul_q4_dyn call of this shape: the split-K slabs, and from 6144 rows
+ * the int8 expansion of int4 weights (a no-op for shapes that need neither; a
+ * capture without the latter runs without). A workspace is allocated per (device, stream) on
  * first need and grows on demand; a growth cannot happen while the stream is
  * being captured into a HIP graph, so callers that capture reserve for their
- * largest shape first. A captured GEMM that splits K keeps the capture
- * stream's slabs, so its graph must not run concurrently with other work that
+ * largest shape first. A captured GEMM that uses one keeps the
+ * capture stream's, so its graph must not run concurrently with other work that
  * uses them (another such graph captured on that stream, or GEMMs on it).
- * GEMMs that do not split K share nothing: K % 128 != 0 runs on zero-padded
+ * Other captured GEMMs share nothing: K % 128 != 0 runs on zero-padded
  * copies of the operands outside capture only, and on a slower kernel with
  * the same results inside. */
 int bh_reserve_workspace(void* stream, uint32_t m, uint32_t kg, uint32_t n);

@@ -57,7 +57,7 @@ from brain_amd import load
 lib = load()
 fake.fake_log.restype = C.c_char_p
 A, CAP = 1 << 20, 0x1000
-kernels = ("pad_rows", "gemm_i8_dma", "gemm_i8_kernel", "splitk_reduce")
+kernels = ("pad_rows", "expand_q4", "gemm_i8_dma", "gemm_i8_kernel", "splitk_reduce")
 def run(stream, m, k, n, q4=False, mem=True, off=0):
     fake.fake_no_memory(0 if mem else 1)
     fake.fake_clear()
@@ -115,3 +115,22 @@ def test_captured_and_per_thread_calls_share_no_padded_copies(dispatch):
                     ("run", CAP, *LONG, dict(off=4, q4=True)), ("run", PER_THREAD, *RAGGED, {}),
                     ("run", CAP, 200, 8192, 1024, dict(q4=True))])
     assert got == [PADDED, STAGED, STAGED, STAGED, STAGED, ["gemm_i8_dma"]]
+
+
+def test_int4_splits(dispatch):
+    """Weights expanded to int8 from 6144 rows where there is a workspace; column ranges where 256x256 tiles would leave most of a round empty;
+    K split where 16 q would not fit one i32 sum (unless there are no slabs for
+    it); padded copies in column ranges from the size their bound allows."""
+    q4 = dict(q4=True)
+    dma = ["gemm_i8_dma"]
+    calls = [
+        (("run", 0, 4096, 4096, 22016, q4), dma * 2), (("run", 0, 4096, 4096, 22016, {}), dma * 2),
+        (("run", 0, 300, 131200, 64, q4), SPLIT), (("run", 0x3000, 300, 131200, 64, dict(q4, mem=False)), STAGED),
+        (("run", CAP, 200, 131200, 64, q4), STAGED), (("run", 0, 4096, 131200, 4096, q4), STAGED),
+        (("run", 0, 300, 9952, 151936, q4), PADDED * 2), (("run", 0, 200, 9960, 151936, q4), STAGED),
+        (("run", 0x3000, 8192, 4096, 11008, dict(q4, mem=False)), dma * 2),
+        (("run", CAP, 8192, 4096, 11008, q4), dma * 2),
+        (("run", 0, 8192, 4096, 11008, q4), ["expand_q4"] + dma * 2),
+        (("reserve", CAP + 0x1000, 8192, 1024, 11008), 0),
+    ]
+    assert dispatch([c for c, _ in calls]) == [want for _, want in calls]

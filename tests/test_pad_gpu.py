@@ -52,6 +52,35 @@ def test_q4_accumulators(gpu, m, k, n):
     assert np.array_equal(got, int8_of(x) @ int4_of(w).T)
 
 
+def gpu_words(g, rows, kw):
+    return torch.randint(-2 ** 31, 2 ** 31, (rows, kw), device="cuda", generator=g, dtype=torch.int64).to(torch.int32)
+
+
+def gpu_int4(w):
+    n = torch.stack([(w >> (4 * b)) & 15 for b in range(8)], -1).reshape(w.shape[0], -1)
+    return torch.where(n > 7, n - 16, n)
+
+
+@pytest.mark.parametrize("m,k,n", [
+    (8192, 256, 1108), (6144, 128, 257),     # expanded to int8
+    (4096, 256, 21000), (5000, 136, 17001),  # column ranges of 256x256 tiles and a rest
+    (300, 131200, 64), (70, 262272, 65),     # K split so that 16 q fit an i32 sum
+    (300, 9952, 151936),                     # padded copies in two column ranges
+    (1152, 10240, 3840),                     # 256x256 tiles split over K
+    (1000, 640, 4000), (1000, 640, 2100), (1000, 648, 3990),  # 128x128 and 64x128 tiles; padded
+])
+def test_q4_large_accumulators(gpu, m, k, n):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m + k + n)
+    x, w = gpu_words(g, m, k // 4), gpu_words(g, n, k // 8)
+    one = torch.ones(max(m, n), device="cuda")
+    got = ops.matmul_q4(x, w, one[:m], one[:n], None, torch.int32, "dyn")
+    rows = torch.arange(m, device="cuda") if m * n * k < 2 ** 36 else torch.randperm(m, device="cuda", generator=g)[:64]
+    xr = x[rows].view(torch.int8).double()
+    for n0 in range(0, n, 16384):  # exact: sums below 2^53
+        assert torch.equal(got[rows, n0:n0 + 16384].double(), xr @ gpu_int4(w[n0:n0 + 16384]).double().t())
+
+
 @pytest.mark.parametrize("reserve", [False, True])
 @pytest.mark.parametrize("q4", [False, True])
 def test_ragged_capture(gpu, q4, reserve):

@@ -79,19 +79,19 @@ def test_q4_dyn_prefill_shapes(gpu, m, k, n):
     check(gpu, m, k, n, "dyn", seed=m + k + n, sample=None if m * n <= 512 * 3072 else 300)
 
 
-# From M=256 with K % 32 == 0 the int4 weights are expanded to int8 and the
-# int8 GEMM runs (here also splitting K: 256x4096x130); below, or with K % 32
-# != 0, the register-staged int4 kernel.
+# K % 128 == 0 (or padded to it): the int4 weights go into the int8 GEMM's tiles
+# (here also splitting K: 256x4096x130), whatever M.
 @pytest.mark.parametrize("m,k,n", [(33, 8, 1), (40, 24, 130), (129, 200, 257), (1, 4096, 5), (300, 200, 64),
                                    (256, 4096, 130), (255, 1024, 96)])
 def test_q4_dyn_edges(gpu, m, k, n):
     check(gpu, m, k, n, "dyn", seed=m + k + n)
 
 
-def test_q4_expanded_gemm_in_a_graph(gpu):
-    """The expansion + int8 GEMM recorded in a HIP graph (its workspaces sized
-    first with bh_reserve_workspace, kg = K/4) replays to the eager bits."""
-    m, k, n = 512, 2048, 384
+@pytest.mark.parametrize("m,k,n", [(512, 2048, 384), (6144, 256, 384)])
+def test_q4_expanded_gemm_in_a_graph(gpu, m, k, n):
+    """A GEMM that splits K, and from 6144 rows the expansion to int8 and its
+    GEMM, recorded in a HIP graph (the workspaces sized first with
+    bh_reserve_workspace, kg = K/4), replay to the eager bits."""
     xq, w4, sx, sw, _ = make(m, k, n, 8)
     d = [dev_u32(xq, gpu), dev_u32(w4, gpu), torch.from_numpy(sx).to(gpu), torch.from_numpy(sw).to(gpu)]
     out = torch.empty(m, n, device=gpu)
