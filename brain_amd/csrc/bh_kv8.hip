@@ -221,12 +221,12 @@ __global__ __launch_bounds__(APT) void paged_decode_apply_i8_kernel(PagedReadArg
     for (uint32_t j_seg = 0; j_seg < t;) {
         const uint32_t j_end = t - j_seg > per_seg ? j_seg + per_seg : t;
         const uint32_t blk0 = j_seg / a.bs;
-        const uint32_t nblk = (j_end - j_seg + a.bs - 1) / a.bs;
+        const uint32_t nblk = (j_end - j_seg - 1) / a.bs + 1;  // (a block size near 2^32 added to the length would wrap)
         __syncthreads();
         for (uint32_t i = threadIdx.x; i < nblk; i += APT)
             tbl[i] = blk0 + i < a.max_bt ? min(a.bt[(uint64_t)b * a.max_bt + blk0 + i], none) : none;
         __syncthreads();
-        const uint32_t nch = (j_end - j_seg + APC - 1) / APC;
+        const uint32_t nch = (j_end - j_seg - 1) / APC + 1;
         // Every load is unconditional, at an address inside the buffers (a
         // load under a branch would be waited for at the join). B4: the four
         // positions lie in one block, so one lookup serves them.

@@ -80,3 +80,33 @@ def test_paged_scores_apply_chunk_edges(gpu, lens, bs, n_kv, group, hd):
     assert np.array_equal(got_s.view(np.uint32).ravel(), ws.view(np.uint32).ravel())
     wc = o.paged_decode_apply_i8(np.where(mask, np.float32(0), probs), pool, bt, lens, sc, nh, group, hd, bs, n_kv * hd, cap)
     assert np.array_equal(got_c.ravel(), np.asarray(wc, np.float32).ravel())
+
+
+@pytest.mark.parametrize("lens,bs,nh,group", [
+    ([5, 200, 129], 2 ** 32 - 1, 4, 2), ([5, 200, 129], 2 ** 32 - 4, 4, 2), ([5, 200, 129], 2 ** 32 - 16, 2, 1),
+])
+def test_paged_sizes_near_the_end_of_32_bits(gpu, lens, bs, nh, group):
+    """One block holds every position; a sum with its size would wrap."""
+    rng = np.random.default_rng(5)
+    batch, hd, n_kv, cap, slots = len(lens), 64, (nh - 1) // group + 1, max(lens), 256
+    bt, ln = np.zeros((batch, 1), np.uint32), np.array(lens, np.uint32)
+    pool = rng.integers(0, 2 ** 32, slots * n_kv * hd // 4, dtype=np.uint32)
+    sc = rng.uniform(0.01, 0.05, slots * n_kv).astype(np.float32)
+    q = rng.standard_normal((batch, nh, hd)).astype(np.float32)
+    probs = rng.random((batch, nh, cap)).astype(np.float32)
+    pre = np.full((batch, nh, cap), 7.0, np.float32)
+    # The oracle with one block of the pool's size and a group of the heads: the same slots.
+    obs, og = slots, min(group, nh)
+    want_s = o.paged_decode_scores_i8(q, pool, bt, lens, sc, pre, nh, og, hd, obs, n_kv * hd, cap, 0.125)
+    want_c = o.paged_decode_apply_i8(probs, pool, bt, lens, sc, nh, og, hd, obs, n_kv * hd, cap)
+    lib, st = load(), torch.cuda.current_stream().cuda_stream
+    d = {k: dev(v.view(np.int32) if v.dtype == np.uint32 else v)
+         for k, v in dict(q=q, probs=probs, pool=pool, sc=sc, bt=bt, ln=ln, s=pre).items()}
+    ctx = torch.empty(batch, nh, hd, device="cuda")
+    shape = (batch, nh, group, hd, bs, n_kv * hd, cap, 1)
+    check(lib.bh_paged_decode_scores_i8(st, d["q"].data_ptr(), d["pool"].data_ptr(), pool.size, d["bt"].data_ptr(),
+                                        d["ln"].data_ptr(), d["sc"].data_ptr(), sc.size, d["s"].data_ptr(), *shape, 0.125))
+    check(lib.bh_paged_decode_apply_i8(st, d["probs"].data_ptr(), d["pool"].data_ptr(), pool.size, d["bt"].data_ptr(),
+                                       d["ln"].data_ptr(), d["sc"].data_ptr(), sc.size, ctx.data_ptr(), *shape))
+    assert np.array_equal(d["s"].cpu().numpy().view(np.uint32).ravel(), np.asarray(want_s, np.float32).view(np.uint32).ravel())
+    assert np.array_equal(ctx.cpu().numpy().view(np.uint32).ravel(), np.asarray(want_c, np.float32).view(np.uint32).ravel())
