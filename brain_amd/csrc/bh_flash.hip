@@ -605,3 +605,17 @@ hipError_t launch_flash_prefill(hipStream_t s, const FlashArgs& a, int hd, bool 
 }
 
 }  // namespace bh
+
+// The kernel alone, with its arguments spelled out (not in the public header:
+// the engine launches it; the tests call this).
+extern "C" int bh_flash_prefill_rows(void* stream, float* q, const void* kc, const void* vc, const float* ks,
+                                     const float* vs, const uint32_t* pos, const uint32_t* seq, const uint32_t* bt,
+                                     uint32_t nh, uint32_t nkv, uint32_t hd, uint32_t rows_per_seq, uint32_t nseq,
+                                     uint32_t max_seq, uint32_t max_bt, uint32_t bs, uint32_t nblk, float scale,
+                                     uint32_t kv8) {
+    if (!nkv || nh % nkv || !bh::flash_ok((int)hd, (int)nh, (int)nkv, (int)max_seq)) return (int)hipErrorInvalidValue;
+    const bh::FlashArgs a{q, kc, vc, ks, vs, pos, seq, (int)nh, (int)nkv, (int)(nh * hd), (int)(nkv * hd),
+                          (int)rows_per_seq, (int)nseq, scale,
+                          bh::KvMap{bt, (int)max_bt, (int)bs, (int)nblk, (int)max_seq}};
+    return (int)bh::launch_flash_prefill((hipStream_t)stream, a, (int)hd, kv8 != 0);
+}

@@ -19,19 +19,9 @@ from brain_amd import load
 pytestmark = pytest.mark.gpu
 
 
-class KvMap(C.Structure):
-    _fields_ = [("bt", C.c_void_p), ("max_bt", C.c_int), ("bs", C.c_int), ("nblk", C.c_int), ("max_seq", C.c_int)]
-
-
-class FlashArgs(C.Structure):
-    _fields_ = [(n, C.c_void_p) for n in ("q", "kc", "vc", "ks", "vs", "pos", "seq")] + \
-               [(n, C.c_int) for n in ("nh", "nkv", "hq", "hkv", "rows_per_seq", "nseq")] + \
-               [("scale", C.c_float), ("map", KvMap)]
-
-
 def flash():
-    fn = getattr(load(), "_ZN2bh20launch_flash_prefillEP12ihipStream_tRKNS_9FlashArgsEib")
-    fn.restype, fn.argtypes = C.c_int, [C.c_void_p, C.POINTER(FlashArgs), C.c_int, C.c_bool]
+    fn = load().bh_flash_prefill_rows
+    fn.restype, fn.argtypes = C.c_int, [C.c_void_p] * 9 + [C.c_uint32] * 9 + [C.c_float, C.c_uint32]
     return fn
 
 
@@ -71,10 +61,9 @@ class Setup:
         pos = torch.arange(p0, p1, device="cuda", dtype=torch.int32).repeat(self.nseq)
         seq = torch.arange(self.nseq, device="cuda", dtype=torch.int32).repeat_interleave(n)
         ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
-        a = FlashArgs(q.data_ptr(), ptr(self.k), ptr(self.v), ptr(self.ks), ptr(self.vs), pos.data_ptr(), seq.data_ptr(),
-                      self.nh, self.nkv, self.nh * self.hd, self.nkv * self.hd, n, self.nseq, self.scale,
-                      KvMap(ptr(self.bt), self.max_bt, self.bs, self.nblk, self.max_seq))
-        rc = flash()(torch.cuda.current_stream().cuda_stream, C.byref(a), self.hd, self.kv8)
+        rc = flash()(torch.cuda.current_stream().cuda_stream, q.data_ptr(), ptr(self.k), ptr(self.v), ptr(self.ks),
+                     ptr(self.vs), pos.data_ptr(), seq.data_ptr(), ptr(self.bt), self.nh, self.nkv, self.hd, n, self.nseq,
+                     self.max_seq, self.max_bt, self.bs, self.nblk, self.scale, self.kv8)
         assert rc == 0
         torch.cuda.synchronize()
         return q
