@@ -107,23 +107,23 @@ __global__ __launch_bounds__(64) void paged_decode_scores_i8_kernel(PagedReadArg
 }
 
 // Scores for head_dim 64 and 128 with 16-byte key rows: one thread per
-// (b, kv head, j) and every query head of the kv head's group. The latency
-// of the slot lookup and of the key row bounds it, so the row's HD / 16 loads
-// all go out together and the group's heads share them (one thread per query
-// head read each row once per head, 16 bytes at a time: 8 sequences of
-// 1024-2048 tokens, 16 heads of 128 over 8 kv heads, 12.0 -> 10.4 us).
-// Two heads run at once so that two of the ordered chains are in flight. q is
-// uniform over the workgroup and comes through scalar loads.
+// (b, set of a kv head's query heads, j). The latency of the slot lookup and of
+// the key row bounds it, so the row's HD / 16 loads all go out together and the
+// set's heads share them. Two heads run at once so that two of the ordered
+// chains are in flight. q is uniform over the workgroup and comes through scalar
+// loads. How many heads a set holds: score_sets.
 template <int HD>
-__global__ __launch_bounds__(64) void paged_decode_scores_i8_group_kernel(PagedReadArgs a,
+__global__ __launch_bounds__(64) void paged_decode_scores_i8_group_kernel(PagedReadArgs a, uint32_t nkvu, uint32_t sets,
+                                                                          uint32_t heads,
                                                                           const float* __restrict__ qall,
                                                                           float* __restrict__ out) {
     const uint32_t nchunk = (a.cap + 63) / 64;
-    const uint32_t nkvu = (a.n_heads + a.group - 1) / a.group;  // kv heads that have queries
-    const uint32_t bk = blockIdx.x / nchunk;
+    const uint32_t bs = blockIdx.x / nchunk, set = bs % sets, bk = bs / sets;
     const uint32_t b = bk / nkvu, kvh = bk % nkvu;
     const uint32_t j = (blockIdx.x % nchunk) * 64 + threadIdx.x;
-    if (j >= a.cap || j >= a.seq_lens[b]) return;
+    const uint32_t h0 = kvh * a.group;  // below n_heads
+    const uint32_t h1 = h0 + min(min(a.group, a.n_heads - h0), (set + 1) * heads);
+    if (h0 + set * heads >= h1 || j >= a.cap || j >= a.seq_lens[b]) return;
     uint64_t slot;
     if (!slot_of(a, b, j, kvh, slot)) return;
     const uint4* p = reinterpret_cast<const uint4*>(a.pool) + (slot * a.kv_stride + (uint64_t)kvh * HD) / 16;
@@ -131,8 +131,7 @@ __global__ __launch_bounds__(64) void paged_decode_scores_i8_group_kernel(PagedR
 #pragma unroll
     for (int i = 0; i < HD / 16; ++i) w[i] = p[i];
     const float qscale = a.scales[slot * (a.kv_stride / HD) + kvh];
-    const uint32_t h1 = min((kvh + 1) * a.group, a.n_heads);
-    for (uint32_t h = kvh * a.group; h < h1; h += 2) {
+    for (uint32_t h = h0 + set * heads; h < h1; h += 2) {
         const bool two = h + 1 < h1;
         const float* q0 = qall + ((uint64_t)b * a.n_heads + h) * HD;
         const float* q1 = two ? q0 + HD : q0;
@@ -151,6 +150,28 @@ __global__ __launch_bounds__(64) void paged_decode_scores_i8_group_kernel(PagedR
         o[0] = acc0 * qscale * a.scale;
         if (two) o[a.cap] = acc1 * qscale * a.scale;
     }
+}
+
+// How many sets the query heads of a kv head are split into. A set of the whole
+// group reads each key row once, but its heads run one pair after another: worth
+// it while the workgroups fill the chip, 2048 of one wave (8 per CU). Scores of 8
+// sequences of 1024-2048 tokens, heads of 128, us (whole group / pairs of heads /
+// one thread per head): 16 heads over 8 kv heads 6.6 / 6.8 / 10.5; 32 over 8 (2048
+// workgroups) 8.4 / 9.7 / 18.0; 64 over 8 12.3 / 15.4 / 32.5; 32 over 2 (512)
+// 17.3 / 9.6 / 15.0; 32 over 1 (256) 28.8 / 9.8 / 11.0, one sequence 28.5 / 4.7 / 4.3.
+uint32_t score_sets(uint64_t blocks, uint32_t group) {
+    const uint64_t pairs = (group - 1) / 2 + 1;
+    return (uint32_t)std::min<uint64_t>(pairs, std::max<uint64_t>(1, 2048 / blocks));
+}
+
+template <int HD>
+void go_scores_group(hipStream_t s, const PagedReadArgs& a, uint32_t batch) {
+    const uint32_t nchunk = (a.cap + 63) / 64, nkvu = (a.n_heads - 1) / a.group + 1;  // kv heads that have queries
+    const uint32_t group = std::min(a.group, a.n_heads);
+    const uint64_t blocks = (uint64_t)batch * nkvu * nchunk;
+    const uint32_t want = score_sets(blocks, group);
+    const uint32_t heads = ((group + want - 1) / want + 1) / 2 * 2, sets = (group + heads - 1) / heads;
+    paged_decode_scores_i8_group_kernel<HD><<<(unsigned)(blocks * sets), 64, 0, s>>>(a, nkvu, sets, heads, a.in, a.out);
 }
 
 // Context: per (b, h, d) the sum over positions j, in order, of
@@ -347,9 +368,8 @@ hipError_t launch_paged_decode_i8(hipStream_t s, bool apply, const PagedReadArgs
         const uint64_t grid = (uint64_t)batch * a.n_heads * nchunk;
         if (grid == 0) return hipSuccess;
         const bool vec = a.hd % 16 == 0 && a.kv_stride % 16 == 0 && (reinterpret_cast<uintptr_t>(a.pool) & 15) == 0;
-        const uint64_t ggrid = (uint64_t)batch * ((a.n_heads + a.group - 1) / a.group) * nchunk;
-        if (vec && a.hd == 128) paged_decode_scores_i8_group_kernel<128><<<(unsigned)ggrid, 64, 0, s>>>(a, a.in, a.out);
-        else if (vec && a.hd == 64) paged_decode_scores_i8_group_kernel<64><<<(unsigned)ggrid, 64, 0, s>>>(a, a.in, a.out);
+        if (vec && a.hd == 128) go_scores_group<128>(s, a, batch);
+        else if (vec && a.hd == 64) go_scores_group<64>(s, a, batch);
         else if (vec) paged_decode_scores_i8_kernel<true><<<(unsigned)grid, 64, 0, s>>>(a);
         else paged_decode_scores_i8_kernel<false><<<(unsigned)grid, 64, 0, s>>>(a);
     } else {

@@ -2,7 +2,7 @@
 wrong: sequence lengths around the 128-position chunk and its multiples, block
 sizes with and without a factor of 4, a table longer than the part staged at a
 time, head_dim below, at and above the 64-wide workgroup, groups of one to
-five heads, and table entries outside the pool. Bit for bit against the
+32 heads, and table entries outside the pool. Bit for bit against the
 oracle, which sums in the same order."""
 import numpy as np
 import pytest
@@ -27,6 +27,8 @@ def dev(a):
     ([300, 64], 4, 1, 2, 256),
     ([2049, 2048, 6001], 1, 1, 2, 64),   # 6001 table entries: three staged parts
     ([1029, 0, 77], 16, 2, 2, 72),
+    ([200, 3], 16, 2, 9, 64), ([70, 513, 1], 32, 1, 32, 128),  # sets of two heads and a rest
+    ([2100] + [2000] * 31, 32, 2, 3, 64), ([1400] * 24, 32, 1, 7, 128),  # of the whole group; of four and three
 ])
 def test_paged_scores_apply_chunk_edges(gpu, lens, bs, n_kv, group, hd):
     rng = np.random.default_rng(sum(lens) + bs)
@@ -84,9 +86,10 @@ def test_paged_scores_apply_chunk_edges(gpu, lens, bs, n_kv, group, hd):
 
 @pytest.mark.parametrize("lens,bs,nh,group", [
     ([5, 200, 129], 2 ** 32 - 1, 4, 2), ([5, 200, 129], 2 ** 32 - 4, 4, 2), ([5, 200, 129], 2 ** 32 - 16, 2, 1),
+    ([5, 200, 129], 256, 4, 2 ** 32 - 1), ([5, 200, 129], 256, 5, 3),
 ])
 def test_paged_sizes_near_the_end_of_32_bits(gpu, lens, bs, nh, group):
-    """One block holds every position; a sum with its size would wrap."""
+    """One block holds every position; a sum with its size or with the group's would wrap."""
     rng = np.random.default_rng(5)
     batch, hd, n_kv, cap, slots = len(lens), 64, (nh - 1) // group + 1, max(lens), 256
     bt, ln = np.zeros((batch, 1), np.uint32), np.array(lens, np.uint32)
