@@ -127,7 +127,8 @@ struct FlashCfg {
 // shared tile, a value that rounds to an infinity in bf16 is lost, and scores
 // below NO_REF leave no weight at all. Here each of them is what the formula
 // gives. Loads are uncoalesced (a lane reads its key's row): this runs for
-// such vectors only.
+// such vectors only. A NaN in the query or a score is NaN in every element and
+// ends it early: once a model has gone to NaN every vector comes here.
 template <bool KV8, int HD>
 __device__ void plain_row(const FlashArgs& p, const uint32_t* tslot, int r, int kh, int h, int lane) {
     float* q = p.q + (size_t)r * p.hq + (size_t)h * HD;
@@ -143,8 +144,22 @@ __device__ void plain_row(const FlashArgs& p, const uint32_t* tslot, int r, int 
         if constexpr (KV8) acc = acc * p.ks[slot * p.nkv + kh];
         return acc * p.scale;
     };
+    bool nan = false;
+#pragma unroll
+    for (int u = 0; u < HD / 64; ++u) nan |= q[lane + 64 * u] != q[lane + 64 * u];
     float mx = -INFINITY;
-    for (int j = lane; j <= pos; j += 64) mx = fmaxf(mx, score(j));
+    if (!__any(nan)) {
+        for (int j = lane; j <= pos; j += 64) {
+            const float s = score(j);
+            nan |= s != s;
+            mx = fmaxf(mx, s);
+        }
+    }
+    if (__any(nan)) {
+#pragma unroll
+        for (int u = 0; u < HD / 64; ++u) q[lane + 64 * u] = __builtin_nanf("");
+        return;
+    }
     mx = xor_max<32>(mx);
     float l = 0.0f, ctx[HD / 64];
 #pragma unroll

@@ -161,7 +161,7 @@ def plain64(s, p1):
 
 
 @pytest.mark.parametrize("hd,group", [(128, 2), (64, 3)])
-@pytest.mark.parametrize("what", ["v_nan", "v_inf", "v_top", "k_low", "k_nan", "vs_inf", "ks_nan"])
+@pytest.mark.parametrize("what", ["v_nan", "v_inf", "v_top", "k_low", "k_nan", "q_nan", "vs_inf", "ks_nan"])
 def test_flash_prefill_values_at_the_ends_of_f32(gpu, what, hd, group):
     """A value that is not finite, or rounds to an infinity in bf16, or scores
     far below any other key, in one cache slot: rows before it do not see it
@@ -177,6 +177,8 @@ def test_flash_prefill_values_at_the_ends_of_f32(gpu, what, hd, group):
         s.v[at, 5] = float("inf")
     elif what == "v_top":
         s.v[at, 5] = torch.finfo(torch.float32).max
+    elif what == "q_nan":
+        s.q[0, 40, 1, 3] = float("nan")
     elif what == "k_nan":
         s.k[at, 5] = float("nan")
     elif what == "k_low":  # row 0 sees this key alone; its score is finite and below -1e34
