@@ -18,7 +18,7 @@
 // f32 MFMA would take 64 cycles per 2048 multiply-adds, against 6 x 32 cycles
 // per 16384 here (3 x 32 with an int8 cache).
 //
-// One workgroup: QG x KS waves; wave (qg, ks) holds 32 query vectors (rows x
+// One workgroup: QG x KS (x DS) waves; wave (qg, ks) holds 32 query vectors (rows x
 // heads of one kv head's group) and walks the key tiles of 32 keys whose
 // index is ks mod KS, with its own running maximum, sum and context (online
 // softmax); at the end the KS parts are merged through LDS in a fixed order.
@@ -35,21 +35,25 @@
 // stored with its keys in the order the lanes hold them.
 //
 // K and V tiles go global -> registers -> (split) -> LDS; the loads of one go
-// out while the other is being multiplied.
+// out while the other is being multiplied (int8 cache), or those of a step
+// before the step before it is through (f32 cache, whose workgroup has its CU to
+// itself: 2000 tokens 153 -> 143 us, and 139 with the third parts of the queries
+// in registers).
 //
 // Measured, 16 query heads over 8 kv heads of 128, one 2000-token prompt /
-// eight of 250: int8 cache 80 / 31 us, f32 cache 175 / 39 us. (The kernel
-// before it, f32 products on the vector units with 32-key partial sums through
-// memory, and its merge: 964 + 138 us for the 2000 tokens, int8.) At 2000
-// tokens the matrix cores are busy 30% of the time and vector instructions
-// issue in 48%: the conversion of the tiles to bf16 and the softmax bound it.
+// eight of 250, K and V in cache: int8 cache 70 / 28 us, f32 cache 139 / 32 us.
+// (The kernel before it, f32 products on the vector units with 32-key partial
+// sums through memory, and its merge: 964 + 138 us for the 2000 tokens, int8.)
+// What bounds it: without the conversion to bf16 parts the f32 cache's kernel
+// takes 16% less, without five of six products 16% less, without either 34%; LDS
+// reads, the softmax and the latency of barriers are the rest.
 // Waves: 2 x 4 for the int8 cache; for the f32 cache, whose split tiles take
-// three times the LDS, 2 x 2 with two workgroups per CU measured 175 / 39 us
-// against 164 / 51 us at 2 x 4, and 12 against 17 us at 64 tokens. KS is part
-// of the result's summation order, so it is one per cache type and not chosen
-// by length. Against 64-bit attention, one 2000-token prompt of normal q, k, v:
-// 1.4e-7 (f32 cache) and 3.0e-7 (int8) in the 2-norm; the f32 kernel 2.2e-7
-// and 3.3e-7.
+// three times the LDS, 2 x 2 (one workgroup per CU by its registers; limited to
+// the registers of two it spills, 191 us), and for few workgroups 1 x 2 x 2 (see
+// SPLIT_D_GRID). KS is part of the result's summation order, so it is one per
+// cache type and not chosen by length. Against 64-bit attention, one 2000-token
+// prompt of normal q, k, v: 1.4e-7 (f32 cache) and 3.0e-7 (int8) in the 2-norm;
+// the f32 kernel 2.2e-7 and 3.3e-7.
 #include <type_traits>
 
 #include "bh_common.h"
@@ -101,22 +105,22 @@ __device__ __forceinline__ v16f mfma(v4i a, v4i b, v16f c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
 }
 
-template <bool KV8, int HD, int QG, int KS>
+template <bool KV8, int HD, int QG, int KS, int DS>
 struct FlashCfg {
-    static constexpr int NT = QG * KS * 64;
+    static constexpr int NT = QG * KS * DS * 64;
+    static constexpr bool DEEP = !KV8;  // the next tiles of K and V both in flight
     static constexpr int KEYS = 32 * KS;               // keys per step
     static constexpr int PARTS = KV8 ? 1 : 3;          // bf16 parts of a cache element
     static constexpr int TILE = 32 * HD * 2;           // bytes of one part of 32 keys
     static constexpr int REGION = KS * PARTS * TILE;   // K, or V, of one step
-    static constexpr bool SEP = 2 * REGION <= 64 * 1024;  // K and V in LDS side by side
+    static constexpr bool SEP = DEEP || 2 * REGION <= 64 * 1024;  // K and V in LDS side by side
     static constexpr int VOFF = SEP ? REGION : 0;
     static constexpr int LDS = SEP ? 2 * REGION : REGION;
-    static constexpr int OREGS = HD / 2;               // context registers per lane
-    static constexpr int MERGE = (KS / 2) * QG * 64 * OREGS * 4;
+    static constexpr int OREGS = HD / 2 / DS;          // context registers per lane
+    static constexpr int MERGE = (KS / 2) * QG * DS * 64 * OREGS * 4;
     static constexpr int NKC = KEYS * HD / 8 / NT;     // 8-element pieces of K per thread
     static constexpr int VB = KEYS * HD / 32;          // 8-key x 4-d blocks of V
     static constexpr int NVB = VB > NT ? VB / NT : 1;  // ... per thread (below VB, the first VB threads)
-    static constexpr int NR = NKC * 2 > NVB * 8 ? NKC * 2 : NVB * 8;
     static_assert(NKC * NT * 8 == KEYS * HD && (VB <= NT || NVB * NT == VB), "whole pieces per thread");
     static_assert(MERGE <= LDS, "the merge fits the tiles' LDS");
 };
@@ -189,19 +193,21 @@ __device__ void plain_row(const FlashArgs& p, const uint32_t* tslot, int r, int 
     for (int u = 0; u < HD / 64; ++u) q[lane + 64 * u] = ctx[u] / l;
 }
 
-template <bool KV8, int HD, int QG, int KS>
-__global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p) {
-    using C = FlashCfg<KV8, HD, QG, KS>;
+template <bool KV8, int HD, int QG, int KS, int DS>
+__global__ __launch_bounds__(QG* KS * DS * 64, HD == 64 ? 2 : 1) void flash_prefill_kernel(FlashArgs p) {
+    using C = FlashCfg<KV8, HD, QG, KS, DS>;
     __shared__ __attribute__((aligned(1024))) uint8_t lds[C::LDS];
-    // The third parts of the queries (one use per key tile) live in LDS: 32
-    // registers fewer at head_dim 128, which is what keeps the kernel from
+    // int8 cache: the third parts of the queries (one use per key tile) live in
+    // LDS: 32 registers fewer at head_dim 128, which is what keeps the kernel from
     // spilling at two waves per SIMD.
-    __shared__ __attribute__((aligned(1024))) uint8_t q3[QG * C::TILE];
-    __shared__ float sml[QG * KS][2][64];
+    __shared__ __attribute__((aligned(1024))) uint8_t q3[KV8 ? QG * C::TILE : 16];
+    __shared__ float sml[QG * KS * DS][2][64];
+    __shared__ uint32_t redo_ds[DS == 1 ? 1 : QG * DS];
     __shared__ __attribute__((aligned(16))) float ksc[KV8 ? C::KEYS : 4], vsc[KV8 ? C::KEYS : 4];
     __shared__ uint32_t tslot[FLASH_MAX_SEQ / 32];
     const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, col = lane & 31;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), qg = wave % QG, ks = wave / QG;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), qg = wave % QG, ks = wave / QG % KS;
+    const int ds = wave / (QG * KS), wd = ds * QG + qg;  // this wave's HD / DS columns of the context
     const int G = p.nh / p.nkv, RW = 32 / G;  // rows per wave
     const int nqb = (p.rows_per_seq + RW * QG - 1) / (RW * QG);
     // The blocks of the latest rows attend the most keys: they start first.
@@ -230,23 +236,25 @@ __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p)
         return r * (HD * 2) + ((HD == 128 ? c ^ (r & 15) : c ^ ((r >> 1) & 7)) << 4);
     };
     const uint8_t* q3w = q3 + qg * C::TILE;
-    v4i qf[HD / 16][2];
+    float4 qraw[HD / 8];
 #pragma unroll
     for (int s = 0; s < HD / 16; ++s) {
-        const float4 lo = *reinterpret_cast<const float4*>(qrow + 16 * s + 8 * half);
-        const float4 hi = *reinterpret_cast<const float4*>(qrow + 16 * s + 8 * half + 4);
-        const float x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-        v4i third;
-        split8(x, qf[s][0], qf[s][1], third);
-        if (ks == 0) *reinterpret_cast<v4i*>(q3 + qg * C::TILE + kchunk(col, 2 * s + half)) = third;
+        qraw[2 * s] = *reinterpret_cast<const float4*>(qrow + 16 * s + 8 * half);
+        qraw[2 * s + 1] = *reinterpret_cast<const float4*>(qrow + 16 * s + 8 * half + 4);
     }
-    __syncthreads();  // tslot, q3
+    // Orders LDS only; the global loads in flight go on.
+    auto barrier = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    barrier();  // tslot
 
     // ---- staging
     constexpr int CPK = HD / 8;  // 16-byte bf16 chunks per key
-    float4 rf[KV8 ? 1 : C::NR];  // K pieces, then V blocks, in flight
-    uint32_t r8[KV8 ? C::NR : 1];
-    float rsc = 0.0f;
+    float4 kf[KV8 ? 1 : C::NKC * 2], vf[KV8 ? 1 : C::NVB * 8];  // K pieces, V blocks in flight
+    uint32_t k8[KV8 ? C::NKC * 2 : 1], v8[KV8 ? C::NVB * 8 : 1];
+    float kscale = 0.0f, vscale = 0.0f;
     // A tile's first cache row of this kv head, as a uniform element offset,
     // and its last visible key. Keys past that repeat it: their weights are
     // zero, and what they multiply is a value that is visible.
@@ -260,11 +268,11 @@ __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p)
         return {(size_t)slot * (uint32_t)p.hkv + (uint32_t)(kh * HD), min(maxpos - 32 * t0, 31)};
     };
     using Elem = std::conditional_t<KV8, uint8_t, float>;
-    auto load_scale = [&](int it, const float* sc) {
+    auto load_scale = [&](int it, const float* sc, float& to) {
         if constexpr (KV8) {
             if (tid < C::KEYS) {
                 const int t0 = min(it * KS + (tid >> 5), maxpos >> 5);
-                rsc = sc[((size_t)tslot[t0] + min(tid & 31, maxpos - 32 * t0)) * p.nkv + kh];
+                to = sc[((size_t)tslot[t0] + min(tid & 31, maxpos - 32 * t0)) * p.nkv + kh];
             }
         }
     };
@@ -282,14 +290,14 @@ __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p)
             const uint32_t o = __umul24((uint32_t)min((kkey + u * KPT) & 31, t.last), (uint32_t)p.hkv) + kcol;
             if constexpr (KV8) {
                 const uint2 v = *reinterpret_cast<const uint2*>(src + o);
-                r8[2 * u] = v.x;
-                r8[2 * u + 1] = v.y;
+                k8[2 * u] = v.x;
+                k8[2 * u + 1] = v.y;
             } else {
-                rf[2 * u] = *reinterpret_cast<const float4*>(src + o);
-                rf[2 * u + 1] = *reinterpret_cast<const float4*>(src + o + 4);
+                kf[2 * u] = *reinterpret_cast<const float4*>(src + o);
+                kf[2 * u + 1] = *reinterpret_cast<const float4*>(src + o + 4);
             }
         }
-        load_scale(it, p.ks);
+        load_scale(it, p.ks, kscale);
     };
     auto store_k = [&]() {
 #pragma unroll
@@ -300,12 +308,12 @@ __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p)
                 v4i w;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const uint32_t cw = r8[2 * u + (i >> 1)];
+                    const uint32_t cw = k8[2 * u + (i >> 1)];
                     w[i] = (int)hi16x2(code_f(cw, 2 * (i & 1)), code_f(cw, 2 * (i & 1) + 1));
                 }
                 *reinterpret_cast<v4i*>(dst) = w;
             } else {
-                const float4 lo = rf[2 * u], hi = rf[2 * u + 1];
+                const float4 lo = kf[2 * u], hi = kf[2 * u + 1];
                 const float x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
                 v4i w0, w1, w2;
                 split8(x, w0, w1, w2);
@@ -315,7 +323,7 @@ __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p)
             }
         }
         if constexpr (KV8)
-            if (tid < C::KEYS) ksc[tid] = rsc;
+            if (tid < C::KEYS) ksc[tid] = kscale;
     };
     // A V block: 8 keys of one k-half of a 16-key step (the keys that half of
     // the lanes holds of the scores: 4h..4h+3 and 8+4h..8+4h+3) x 4 d.
@@ -330,8 +338,8 @@ __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p)
             const Elem* src = static_cast<const Elem*>(p.vc) + t.base;
             const int k0 = 16 * ((oct >> 1) & 1) + 4 * (oct & 1);
             auto at = [&](int j, const Elem* v) {
-                if constexpr (KV8) r8[8 * u + j] = *reinterpret_cast<const uint32_t*>(v);
-                else rf[8 * u + j] = *reinterpret_cast<const float4*>(v);
+                if constexpr (KV8) v8[8 * u + j] = *reinterpret_cast<const uint32_t*>(v);
+                else vf[8 * u + j] = *reinterpret_cast<const float4*>(v);
             };
             if (t.last == 31) {  // a uniform row stride: one lane offset for the eight loads
                 const uint32_t o = __umul24((uint32_t)k0, (uint32_t)p.hkv) + 4 * dg;
@@ -343,7 +351,7 @@ __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p)
                     at(j, src + (__umul24((uint32_t)min(k0 + (j < 4 ? j : 4 + j), t.last), (uint32_t)p.hkv) + 4 * dg));
             }
         }
-        load_scale(it, p.vs);
+        load_scale(it, p.vs, vscale);
     };
     // LDS: V^T part t of tile w: lines of 256 bytes hold 4 d x 32 keys; the
     // chunk of 8 keys (octet o) of d at slot (4 (d % 4) + o) ^ (line & 15) of
@@ -362,9 +370,9 @@ __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p)
                 float x[8];
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
-                    if constexpr (KV8) x[j] = code_f(r8[8 * u + j], e);
+                    if constexpr (KV8) x[j] = code_f(v8[8 * u + j], e);
                     else {
-                        const float4 v = rf[8 * u + j];
+                        const float4 v = vf[8 * u + j];
                         x[j] = e == 0 ? v.x : e == 1 ? v.y : e == 2 ? v.z : v.w;
                     }
                 }
@@ -381,28 +389,34 @@ __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p)
             }
         }
         if constexpr (KV8)
-            if (tid < C::KEYS) vsc[tid] = rsc;
+            if (tid < C::KEYS) vsc[tid] = vscale;
     };
-    // Orders LDS only; the global loads in flight go on.
-    auto barrier = [&]() {
-        __builtin_amdgcn_sched_barrier(0);
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        __builtin_amdgcn_sched_barrier(0);
-    };
-
-    v16f o[HD / 32];
+    constexpr int OJ = HD / 32 / DS;
+    v16f o[OJ];
 #pragma unroll
-    for (int j = 0; j < HD / 32; ++j)
+    for (int j = 0; j < OJ; ++j)
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[j][e] = 0.0f;
     const float c2 = p.scale * 1.44269504088896341f;
     float m = NO_REF, l = 0.0f;  // l: this half's keys only
 
     load_k(0);
+    if constexpr (C::DEEP) load_v(0);
+    v4i qf[HD / 16][2], qf3[KV8 ? 1 : HD / 16];
+#pragma unroll
+    for (int s = 0; s < HD / 16; ++s) {
+        const float4 lo = qraw[2 * s], hi = qraw[2 * s + 1];
+        const float x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+        v4i third;
+        split8(x, qf[s][0], qf[s][1], third);
+        if constexpr (!KV8) qf3[s] = third;
+        else if (ks == 0) *reinterpret_cast<v4i*>(q3 + qg * C::TILE + kchunk(col, 2 * s + half)) = third;
+    }
     for (int it = 0; it < niter; ++it) {
         if constexpr (!C::SEP) barrier();  // the last step's V has been read
         store_k();
-        load_v(it);
+        if constexpr (!C::DEEP) load_v(it);
+        else if (it + 1 < niter) load_k(it + 1);
         barrier();
         const int j0 = it * C::KEYS + 32 * ks;
         const bool live = j0 <= wmaxpos;  // wave-uniform
@@ -417,8 +431,8 @@ __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p)
             for (int t = 0; t < HD / 16; ++t) {
                 const uint8_t* src = kb + kchunk(col, 2 * t + half);
                 const v4i k1 = *reinterpret_cast<const v4i*>(src);
-                const v4i qt = *reinterpret_cast<const v4i*>(q3w + kchunk(col, 2 * t + half));
                 if constexpr (KV8) {
+                    const v4i qt = *reinterpret_cast<const v4i*>(q3w + kchunk(col, 2 * t + half));
                     s = mfma(k1, qt, s);
                     s = mfma(k1, qf[t][1], s);
                     s = mfma(k1, qf[t][0], s);
@@ -426,7 +440,7 @@ __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p)
                     const v4i k2 = *reinterpret_cast<const v4i*>(src + C::TILE);
                     const v4i k3 = *reinterpret_cast<const v4i*>(src + 2 * C::TILE);
                     s = mfma(k3, qf[t][0], s);
-                    s = mfma(k1, qt, s);
+                    s = mfma(k1, qf3[t], s);
                     s = mfma(k2, qf[t][1], s);
                     s = mfma(k2, qf[t][0], s);
                     s = mfma(k1, qf[t][1], s);
@@ -464,7 +478,7 @@ __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p)
                 const float alpha = __builtin_amdgcn_exp2f(m - mn);  // 1 where the reference stays
                 l = l * alpha;
 #pragma unroll
-                for (int j = 0; j < HD / 32; ++j)
+                for (int j = 0; j < OJ; ++j)
 #pragma unroll
                     for (int e = 0; e < 16; ++e) o[j][e] = o[j][e] * alpha;
                 m = mn;
@@ -479,7 +493,10 @@ __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p)
         }
         if constexpr (!C::SEP) barrier();  // every wave has read this step's K
         store_v();
-        if (it + 1 < niter) load_k(it + 1);
+        if (it + 1 < niter) {
+            if constexpr (C::DEEP) load_v(it + 1);
+            else load_k(it + 1);
+        }
         barrier();
         if (live) {
             if constexpr (KV8) {
@@ -502,8 +519,8 @@ __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p)
                 split8(x, pf[t][0], pf[t][1], pf[t][2]);
             }
 #pragma unroll
-            for (int j = 0; j < HD / 32; ++j) {
-                const int d = 32 * j + col;
+            for (int j = 0; j < OJ; ++j) {
+                const int d = 32 * (ds * OJ + j) + col;
                 const uint8_t* src[2] = {vb + vchunk(d >> 2, d & 3, half), vb + vchunk(d >> 2, d & 3, 2 + half)};
                 if constexpr (KV8) {
 #pragma unroll
@@ -545,25 +562,25 @@ __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p)
 #pragma unroll
     for (int w = KS / 2; w >= 1; w /= 2) {
         barrier();
-        float4* om = reinterpret_cast<float4*>(lds) + (size_t)((ks % w) * QG + qg) * 64 * (HD / 8) + lane;
+        float4* om = reinterpret_cast<float4*>(lds) + (size_t)((ks % w) * QG * DS + wd) * 64 * (C::OREGS / 4) + lane;
         if (ks >= w && ks < 2 * w) {
 #pragma unroll
-            for (int j = 0; j < HD / 32; ++j)
+            for (int j = 0; j < OJ; ++j)
 #pragma unroll
                 for (int e4 = 0; e4 < 4; ++e4)
                     om[(4 * j + e4) * 64] = make_float4(o[j][4 * e4], o[j][4 * e4 + 1], o[j][4 * e4 + 2], o[j][4 * e4 + 3]);
-            sml[(ks % w) * QG + qg][0][lane] = m;
-            sml[(ks % w) * QG + qg][1][lane] = l;
+            sml[(ks % w) * QG * DS + wd][0][lane] = m;
+            sml[(ks % w) * QG * DS + wd][1][lane] = l;
         }
         barrier();
         if (ks < w) {
-            const float m2 = sml[(ks % w) * QG + qg][0][lane], l2 = sml[(ks % w) * QG + qg][1][lane];
+            const float m2 = sml[(ks % w) * QG * DS + wd][0][lane], l2 = sml[(ks % w) * QG * DS + wd][1][lane];
             const float mn = fmaxf(m, m2);
             const float a1 = __builtin_amdgcn_exp2f(m - mn), a2 = __builtin_amdgcn_exp2f(m2 - mn);
             m = mn;
             l = l * a1 + l2 * a2;
 #pragma unroll
-            for (int j = 0; j < HD / 32; ++j)
+            for (int j = 0; j < OJ; ++j)
 #pragma unroll
                 for (int e4 = 0; e4 < 4; ++e4) {
                     const float4 v = om[(4 * j + e4) * 64];
@@ -574,49 +591,77 @@ __global__ __launch_bounds__(QG* KS * 64) void flash_prefill_kernel(FlashArgs p)
                 }
         }
     }
+    uint32_t redo = 0;
     if (ks == 0) {
         const float inv = 1.0f / (l + xor_lane<32>(l));
         float z = 0.0f;  // NaN once a context element is not finite
 #pragma unroll
-        for (int j = 0; j < HD / 32; ++j)
+        for (int j = 0; j < OJ; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 o[j][e] = o[j][e] * inv;
                 z = __builtin_fmaf(o[j][e], 0.0f, z);
             }
         const unsigned long long bad = __ballot(qlive && z != 0.0f);
-        uint32_t redo = (uint32_t)bad | (uint32_t)(bad >> 32);  // by col: a vector's two halves
+        redo = (uint32_t)bad | (uint32_t)(bad >> 32);  // by col: a vector's two halves
+    }
+    if constexpr (DS > 1) {  // ... and its DS parts
+        if (ks == 0 && lane == 0) redo_ds[wd] = redo;
+        barrier();
+        redo = 0;
+#pragma unroll
+        for (int i = 0; i < DS; ++i) redo |= (uint32_t)__builtin_amdgcn_readfirstlane((int)redo_ds[i * QG + qg]);
+    }
+    if (ks == 0) {
         if (qlive && !((redo >> col) & 1u)) {
 #pragma unroll
-            for (int j = 0; j < HD / 32; ++j)
+            for (int j = 0; j < OJ; ++j)
 #pragma unroll
                 for (int e4 = 0; e4 < 4; ++e4)
-                    *reinterpret_cast<float4*>(qrow + 32 * j + 8 * e4 + 4 * half) =
+                    *reinterpret_cast<float4*>(qrow + 32 * (ds * OJ + j) + 8 * e4 + 4 * half) =
                         make_float4(o[j][4 * e4], o[j][4 * e4 + 1], o[j][4 * e4 + 2], o[j][4 * e4 + 3]);
         }
         // Live columns only (bad is 0 elsewhere); their queries are not yet
         // overwritten.
-        for (; redo; redo &= redo - 1u) {
+        for (; ds == 0 && redo; redo &= redo - 1u) {
             const int c = __ffs(redo) - 1, i = qg * RW + c / G;
             plain_row<KV8, HD>(p, tslot, r0 + i, kh, kh * G + c % G, lane);
         }
     }
 }
 
-template <bool KV8, int HD, int QG, int KS>
-hipError_t go(hipStream_t s, const FlashArgs& a) {
-    const int rb = 32 / (a.nh / a.nkv) * QG;
-    const unsigned grid = (unsigned)((a.rows_per_seq + rb - 1) / rb * a.nseq * a.nkv);
-    flash_prefill_kernel<KV8, HD, QG, KS><<<grid, QG * KS * 64, 0, s>>>(a);
+// Up to this many workgroups of 2 x 2 waves, half the chip, the f32 cache's
+// kernel is a serial chain in each: half the rows per workgroup then, and two
+// waves that each make the whole scores and half of the context's columns (the
+// same bits). 16 heads over 8 of 128, us, 2 x 2 / 1 x 2 x 2: 64 tokens 10.2 / 9.0,
+// 128 14.0 / 12.5, 200 19.4 / 18.7, 512 (128 workgroups) 36.9 / 33.6; 1000
+// (256) 67 / 70, eight sequences of 128 (256) 14.9 / 21.3: more than 256
+// workgroups of the second kind take turns on the CUs.
+constexpr unsigned SPLIT_D_GRID = 128;
+
+template <bool KV8, int HD, int QG, int KS, int DS>
+hipError_t launch(hipStream_t s, const FlashArgs& a, unsigned grid) {
+    flash_prefill_kernel<KV8, HD, QG, KS, DS><<<grid, QG * KS * DS * 64, 0, s>>>(a);
     return hipGetLastError();
+}
+
+template <bool KV8, int HD>
+hipError_t go(hipStream_t s, const FlashArgs& a) {
+    auto grid = [&](int qg) -> unsigned {
+        const int rb = 32 / (a.nh / a.nkv) * qg;
+        return (unsigned)((a.rows_per_seq + rb - 1) / rb * a.nseq * a.nkv);
+    };
+    if constexpr (KV8) return launch<true, HD, 2, 4, 1>(s, a, grid(2));
+    else if (grid(2) <= SPLIT_D_GRID) return launch<false, HD, 1, 2, 2>(s, a, grid(1));
+    else return launch<false, HD, 2, 2, 1>(s, a, grid(2));
 }
 
 }  // namespace
 
 hipError_t launch_flash_prefill(hipStream_t s, const FlashArgs& a, int hd, bool kv8) {
     if (a.rows_per_seq <= 0 || a.nseq <= 0) return hipSuccess;
-    if (hd == 128) return kv8 ? go<true, 128, 2, 4>(s, a) : go<false, 128, 2, 2>(s, a);
-    return kv8 ? go<true, 64, 2, 4>(s, a) : go<false, 64, 2, 2>(s, a);
+    if (hd == 128) return kv8 ? go<true, 128>(s, a) : go<false, 128>(s, a);
+    return kv8 ? go<true, 64>(s, a) : go<false, 64>(s, a);
 }
 
 }  // namespace bh

@@ -134,9 +134,11 @@ def test_flash_prefill_keeps_the_bits_of_a_product(gpu):
 
 
 @pytest.mark.parametrize("kv8", [False, True])
-@pytest.mark.parametrize("hd,group", [(128, 2), (64, 5)])
-def test_flash_prefill_chunking_gives_the_same_bits(gpu, kv8, hd, group):
-    s = Setup(2, 300, 2, group, hd, kv8, True, seed=9)
+@pytest.mark.parametrize("hd,group,nkv", [(128, 2, 2), (64, 5, 2), (128, 2, 8), (64, 1, 16)])
+def test_flash_prefill_chunking_gives_the_same_bits(gpu, kv8, hd, group, nkv):
+    """With 8 and 16 kv heads the whole prompt takes the workgroups of twice the
+    rows (f32 cache, above 128 of them), the chunks those of split columns."""
+    s = Setup(2, 300, nkv, group, hd, kv8, True, seed=9)
     whole = s.run(0, 300)
     cuts = [0, 1, 2, 35, 64, 191, 300]
     parts = torch.cat([s.run(a, b) for a, b in zip(cuts, cuts[1:])], 1)
