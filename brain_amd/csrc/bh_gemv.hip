@@ -1232,11 +1232,15 @@ __global__ __launch_bounds__(256) void gemv_i8_part_kernel(const uint8_t* xq, co
     if (row < m) parts[((int64_t)blockIdx.y * m + row) * n + col] = s;
 }
 
-// Whether launch_gemv_i8_parts takes a shape: at most 16 rows, whole K chunks
-// per wave, and few enough column groups that the split fills idle CUs.
+// Whether launch_gemv_i8_parts takes a shape: at most 16 rows, a whole number
+// of 64-byte K chunks per wave (K % 1024 == 0) and at most 8 (a wave has them all
+// in flight, 64 registers), and few enough column groups that the split fills
+// idle CUs. 8 rows, the whole K / in quarters, N = 1024: K = 2048 4.6 / 3.9 us,
+// 4096 5.7 / 4.0, 5120 7.0 / 4.0, 8192 8.8 / 4.0; N = 2048: 4.6 / 3.9, 6.2 / 4.4,
+// 7.2 / 4.8, 9.2 / 5.5.
 bool gemv_parts_ok(int m, int kg, int n) {
     const int chunks = kg * 4 / 64;
-    return m >= 1 && m <= 16 && kg % 16 == 0 && chunks % 16 == 0 && chunks >= 32 && chunks <= 64 && n % 16 == 0 &&
+    return m >= 1 && m <= 16 && kg % 16 == 0 && chunks % 16 == 0 && chunks >= 32 && chunks <= 128 && n % 16 == 0 &&
            n / 16 <= 128;
 }
 // xq and wq 16-byte aligned; parts [4][m][n].
@@ -1247,6 +1251,10 @@ hipError_t launch_gemv_i8_parts(hipStream_t s, const uint32_t* xq, const uint32_
         case 2: gemv_i8_part_kernel<2><<<grid, 256, 0, s>>>(x, w, m, kg * 4, n, parts); break;
         case 3: gemv_i8_part_kernel<3><<<grid, 256, 0, s>>>(x, w, m, kg * 4, n, parts); break;
         case 4: gemv_i8_part_kernel<4><<<grid, 256, 0, s>>>(x, w, m, kg * 4, n, parts); break;
+        case 5: gemv_i8_part_kernel<5><<<grid, 256, 0, s>>>(x, w, m, kg * 4, n, parts); break;
+        case 6: gemv_i8_part_kernel<6><<<grid, 256, 0, s>>>(x, w, m, kg * 4, n, parts); break;
+        case 7: gemv_i8_part_kernel<7><<<grid, 256, 0, s>>>(x, w, m, kg * 4, n, parts); break;
+        case 8: gemv_i8_part_kernel<8><<<grid, 256, 0, s>>>(x, w, m, kg * 4, n, parts); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

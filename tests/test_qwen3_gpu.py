@@ -378,3 +378,19 @@ def test_qwen3_0_6b_fused_decode_matches_unfused(gpu, batch, kv_int8):
         e.close()
     assert (out[0][0] == out[1][0]).all()
     assert np.array_equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("d_model,d_ff,batch", [(1024, 2048, 5), (1024, 5120, 16), (2048, 6144, 8), (1024, 7168, 7), (256, 8192, 12)])
+def test_decode_projections_split_over_k_are_bit_identical(gpu, d_model, d_ff, batch):
+    """At 5 to 16 rows a down projection of K = 2048 to 8192 leaves K-quarter
+    sums that the next norm adds, against whole sums."""
+    cfg = dict(SMALL, vocab=256, d_model=d_model, d_ff=d_ff)
+    w = scaled_weights(cfg, 3)
+    prompts = np.random.default_rng(3).integers(0, 256, (batch, 9)).astype(np.uint32)
+    out = []
+    for unfused in (False, True):
+        e = engine_for(cfg, w, batch, 24)
+        out.append((e.generate(prompts, 6, eager=unfused, unfused=unfused), e.logits()))
+        e.close()
+    assert (out[0][0] == out[1][0]).all()
+    assert np.array_equal(out[0][1].view(np.uint32), out[1][1].view(np.uint32))
