@@ -51,7 +51,6 @@ hipError_t launch_gemm_i8_noalloc(hipStream_t s, const uint32_t* xq, const uint3
                                   size_t* need_bytes);
 size_t noalloc_scratch_bytes();
 size_t gemm_q4_expand_ints(int m, int k, int n);
-size_t gemm_pad_workspace_ints(int m, int kg, int n);
 hipError_t launch_gemv_i8_gated(hipStream_t s, const uint32_t* xq, const uint32_t* wq, const float* sx,
                                 const float* sw, const float* gate, int gate_stride, int gate_col, float* out, int m,
                                 int kg, int n);

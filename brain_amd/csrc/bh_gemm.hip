@@ -1302,7 +1302,7 @@ static int column_split(int m, int kg, int n, const TileChoice& tc, bool dma) {
 // ---------------------------------------------------------------- padded operands
 // The DMA kernel reads whole 128-byte K stages from 16-byte aligned rows.
 // Operands that are not so (K % 128 != 0, or a pointer off by a word) are
-// first copied to the stream's workspace (slot 1) with their rows zero-padded
+// first copied to the stream's workspace (WS_PAD) with their rows zero-padded
 // to a multiple of 128 bytes (the zeros add nothing to an exact integer sum);
 // the copy is one launch over both operands at memory speed, and the GEMM then
 // runs the tiles of an aligned shape. The register-staged kernel instead loads
